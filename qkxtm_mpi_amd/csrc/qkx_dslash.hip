@@ -422,18 +422,6 @@ __device__ __forceinline__ void epilogue(const Epi &e, const Cx<T> R[12], const 
     }
 }
 
-// Site order of the hop kernels.  Plain: checkerboard index order (x fastest,
-// then y, z, t).  Blocked: x, then yb rows of y, then tb slices of t, then z,
-// then the next y block, then the next t block, so a site's +-y, +-z and +-t
-// neighbours (and the backward links they carry) are reused after about
-// L0 yb tb sites instead of a whole t slice; yb and tb are chosen on the
-// host so that this reuse window stays well inside one XCD's L2.
-struct HopTrav {
-    int on;        // 0: plain order
-    int yb, tb, nyb;
-    FastDiv dyb, dtb, dnyb;
-};
-
 template <class SIn, class SOut, class SAux, class G, int NEPI = QKX_MAX_RHS>
 struct HopArgs {
     Geom g;
@@ -517,64 +505,6 @@ __device__ __forceinline__ void hop_unit(const Geom &g, int par_out, int nblk8, 
         p = (o >= vhn) ? 1 : 0;
         u = o - p * vhn;
     }
-}
-
-// Checkerboard indices of the 8 neighbours of (p, cb) in the other parity,
-// in the order +x -x +y -y +z -z +t -t, and whether the t hops wrap.
-struct HopSite {
-    int nb[8];
-    bool tw_p, tw_m;
-};
-__device__ __forceinline__ HopSite hop_site_at(const Geom &g, int p, int cb, int xh, int y, int z, int t)
-{
-    HopSite h;
-    const int L0 = g.L[0], L1 = g.L[1], L2 = g.L[2], L3 = g.L[3];
-    const int row = cb - xh;   // Lh0 * (y + L1 (z + L2 t))
-    const int x = 2 * xh + ((p + y + z + t) & 1);
-    const int xp = (x + 1 == L0) ? 0 : x + 1;
-    const int xm = (x == 0) ? L0 - 1 : x - 1;
-    h.nb[0] = (xp >> 1) + row;
-    h.nb[1] = (xm >> 1) + row;
-    h.nb[2] = cb + g.Lh0 * ((y + 1 == L1) ? -(L1 - 1) : 1);
-    h.nb[3] = cb + g.Lh0 * ((y == 0) ? (L1 - 1) : -1);
-    const int LY = L1 * g.Lh0;
-    h.nb[4] = cb + ((z + 1 == L2) ? -(L2 - 1) * LY : LY);
-    h.nb[5] = cb + ((z == 0) ? (L2 - 1) * LY : -LY);
-    const int LZ = L2 * LY;
-    h.tw_p = (t + 1 == L3);
-    h.tw_m = (t == 0);
-    h.nb[6] = cb + (h.tw_p ? -(L3 - 1) * LZ : LZ);
-    h.nb[7] = cb + (h.tw_m ? (L3 - 1) * LZ : -LZ);
-    return h;
-}
-
-__device__ __forceinline__ HopSite hop_site(const Geom &g, int p, int cb)
-{
-    const int rest = fdiv(cb, g.dLh0);
-    const int xh = cb - rest * g.Lh0;
-    const int zt = fdiv(rest, g.dL1);
-    const int y = rest - zt * g.L[1];
-    const int t = fdiv(zt, g.dL2);
-    const int z = zt - t * g.L[2];
-    return hop_site_at(g, p, cb, xh, y, z, t);
-}
-
-// The v-th site of parity p in the walk order of tr: its checkerboard index
-// cb and its neighbours.  v < Vh.
-__device__ __forceinline__ HopSite hop_site_walk(const Geom &g, const HopTrav &tr, int p, int v, int &cb)
-{
-    if (!tr.on) {
-        cb = v;
-        return hop_site(g, p, v);
-    }
-    const int q1 = fdiv(v, g.dLh0), xh = v - q1 * g.Lh0;
-    const int q2 = fdiv(q1, tr.dyb), yi = q1 - q2 * tr.yb;
-    const int q3 = fdiv(q2, tr.dtb), ti = q2 - q3 * tr.tb;
-    const int q4 = fdiv(q3, g.dL2), z = q3 - q4 * g.L[2];
-    const int tbk = fdiv(q4, tr.dnyb), ybk = q4 - tbk * tr.nyb;
-    const int y = ybk * tr.yb + yi, t = tbk * tr.tb + ti;
-    cb = xh + g.Lh0 * (y + g.L[1] * (z + g.L[2] * t));
-    return hop_site_at(g, p, cb, xh, y, z, t);
 }
 
 // What a hop thread does with its result.  StoreFin: write it (and, on
@@ -1544,33 +1474,12 @@ const HopShape *g_force = nullptr;  // set while the tuner times a candidate
 bool g_tuning = false;
 thread_local int g_no_tune = 0;     // callers that must not allocate (scratch fields) set this
 
-// Blocked walk for a launch moving site_bytes per output site: rows of y in
-// blocks of up to 8, and as many t slices per block (up to 8, dividing L3)
-// as keep one z plane of a block -- the traffic between a site's use as a
-// +z neighbour and its use as a -z neighbour -- under 1.5 MB, well inside
-// the 4 MB L2 of one XCD.
-constexpr double kTravWindow = 1.5e6;
 constexpr double kTravAutoBytes = 700.0;   // FP64 full-lattice hops move 768-1152 B per site
 HopTrav hop_trav(const Geom &g, int par_out, double site_bytes)
 {
-    HopTrav tr{};
-    if (!g_site_order) return tr;
-    if (g_site_order == 2 && !(par_out < 0 && site_bytes >= kTravAutoBytes)) return tr;
-    int yb = 1;
-    for (int d = 2; d <= 8; d++)
-        if (g.L[1] % d == 0) yb = d;
-    const double row = (par_out < 0 ? g.L[0] : g.Lh0) * site_bytes;
-    int tb = 1;
-    for (int d = 2; d <= 8; d++)
-        if (g.L[3] % d == 0 && row * yb * d <= kTravWindow) tb = d;
-    tr.yb = yb;
-    tr.tb = tb;
-    tr.nyb = g.L[1] / yb;
-    tr.dyb = make_fastdiv(yb);
-    tr.dtb = make_fastdiv(tb);
-    tr.dnyb = make_fastdiv(tr.nyb);
-    tr.on = (yb > 1 || tb > 1) ? 1 : 0;
-    return tr;
+    if (!g_site_order) return HopTrav{};
+    if (g_site_order == 2 && !(par_out < 0 && site_bytes >= kTravAutoBytes)) return HopTrav{};
+    return blocked_walk(g, (par_out < 0 ? g.L[0] : g.Lh0) * site_bytes);
 }
 
 template <class S, class G, int B, class Fin = StoreFin>

@@ -11,342 +11,407 @@
 // is 4 channels, one per spin).  It is linear in its input, so it is a fixed
 // linear operator once trained.
 //
-// Feature fields: float2 (one complex) per (channel, colour, site), component
-// k = channel*3 + colour at base[k*V + s], s the parity-blocked site index of
-// the spinor/gauge layout.  Weights are W[9][cout][cin] complex; the master
-// copy is FP32, inference reads a BF16 copy (FP32 accumulation).
-#include "qkx_internal.h"
-#include "qkx_core.h"
-#include <algorithm>
+// Hidden-channel fields: component k = channel*3 + colour, two per float4 (see
+// Hid), over the parity-blocked site index of the spinor/gauge layout; the
+// 4-channel fields are spinors.  Weights are W[9][cout][cin] complex; the
+// master copy is FP32, inference reads a BF16 copy (FP32 accumulation).
+#include "qkx_net.h"
 #include <chrono>
 #include <cmath>
-#include <type_traits>
 #include <vector>
-
-struct qkx_net_s {
-    int ch;
-    int n1, n2;            // complex weights of layer 1 ([9][ch][4]) and layer 2 ([9][4][ch])
-    float2 *w;             // FP32 master weights, W1 then W2
-    uint32_t *wb;          // BF16 copies (re in the low half, im in the high half)
-    double2 *grad;         // accumulated gradient (dL/dRe + i dL/dIm)
-    float2 *m, *v;         // Adam moments
-    double *loss;          // accumulated loss
-    int step;              // Adam steps taken
-    int bf16;              // inference/training forward reads the BF16 copy
-    int L[4];              // lattice of the work buffers
-    float2 *fin, *fh, *fout, *gout, *gh;   // work buffers: 4ch, ch, 4ch, 4ch, ch channels
-    double *part;
-    int part_cap;
-    float2 *weo;           // even-odd weight tables (forward, then adjoint), see eo_weights_kernel
-    float2 *ehid;          // even-odd hidden channels on the odd sites, [3 ch][Vh][nrhs]
-    size_t ehid_cap;       // float2 entries of ehid
-    size_t ehid_limit;     // bound on ehid (float2 entries); 0: kEoHiddenCap
-};
 
 namespace {
 
-constexpr int kT = 256;
-
-__device__ __forceinline__ uint32_t f2bf(float f)
-{
-    uint32_t u = __float_as_uint(f);
-    u += 0x7fffu + ((u >> 16) & 1u);   // round to nearest even
-    return u >> 16;
-}
-__device__ __forceinline__ float bf2f(uint32_t h) { return __uint_as_float(h << 16); }
-
-__device__ __forceinline__ int rev_path(int p) { return p == 0 ? 0 : (((p - 1) & 1) == 0 ? p + 1 : p - 1); }
-
-// coordinates of parity-blocked site s
-__device__ __forceinline__ void coords_of(const Geom &g, int s, int x[4])
-{
-    const int par = s >= g.Vh ? 1 : 0;
-    const int cb = s - par * g.Vh;
-    const int xh = cb % g.Lh0;
-    const int rest = cb / g.Lh0;
-    x[1] = rest % g.L[1];
-    const int zt = rest / g.L[1];
-    x[2] = zt % g.L[2];
-    x[3] = zt / g.L[2];
-    x[0] = 2 * xh + ((par + x[1] + x[2] + x[3]) & 1);
-}
-__device__ __forceinline__ int site_of(const Geom &g, const int x[4])
-{
-    const int par = (x[0] + x[1] + x[2] + x[3]) & 1;
-    return par * g.Vh + (x[0] >> 1) + g.Lh0 * (x[1] + g.L[1] * (x[2] + g.L[2] * x[3]));
-}
-
-// path p at site x: neighbour site, link site, dagger flag and boundary sign
-struct Hop {
-    int sn, sl;
-    bool dag;
-    float sign;
-};
-__device__ __forceinline__ Hop path_hop(const Geom &g, const int x[4], int s, int p)
-{
-    Hop h{s, s, false, 1.0f};
-    if (p == 0) return h;
-    const int mu = (p - 1) >> 1;
-    int y[4] = {x[0], x[1], x[2], x[3]};
-    if (((p - 1) & 1) == 0) {   // forward
-        y[mu] = (x[mu] + 1 == g.L[mu]) ? 0 : x[mu] + 1;
-        h.sn = site_of(g, y);
-        h.sl = s;
-        h.dag = false;
-        if (mu == 3 && x[3] + 1 == g.L[3]) h.sign = (float)g.bc;
-    } else {                    // backward
-        y[mu] = (x[mu] == 0) ? g.L[mu] - 1 : x[mu] - 1;
-        h.sn = site_of(g, y);
-        h.sl = h.sn;
-        h.dag = true;
-        if (mu == 3 && x[3] == 0) h.sign = (float)g.bc;
-    }
-    return h;
-}
-
-__device__ __forceinline__ void load_link(const GaugeF18 &U, const Hop &h, int p, Cx<float> u[9])
-{
-    const int mu = (p - 1) >> 1;
-    Cx<float> l[9];
-    U.load(mu, h.sl, l);
-#pragma unroll
-    for (int r = 0; r < 3; r++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const Cx<float> e = h.dag ? Cx<float>{l[c * 3 + r].re, -l[c * 3 + r].im} : l[r * 3 + c];
-            u[r * 3 + c] = {h.sign * e.re, h.sign * e.im};
-        }
-}
-
-__device__ __forceinline__ void matvec(const Cx<float> u[9], const Cx<float> v[3], Cx<float> o[3])
-{
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-        Cx<float> a = cmul(u[r * 3], v[0]);
-        a = a + cmul(u[r * 3 + 1], v[1]);
-        a = a + cmul(u[r * 3 + 2], v[2]);
-        o[r] = a;
-    }
-}
-
-__device__ __forceinline__ Cx<float> ldf(const float2 *f, int k, int V, int s)
-{
-    const float2 v = f[(size_t)k * V + s];
-    return {v.x, v.y};
-}
-
-// One PTC layer (CIN -> COUT channels), or the adjoint of the layer whose
-// weights are given (ADJ: A[p][a][b] = conj(W[rev p][b][a]), W of shape
-// [9][CIN][COUT]).  One thread per site; the input channels are streamed so
-// that only the COUT x 3 accumulators stay live.
-template <int CIN, int COUT, bool ADJ, bool BF>
-__global__ __launch_bounds__(kT) void ptc_kernel(const float2 *__restrict__ in, float2 *__restrict__ out, GaugeF18 U,
-                                                 Geom g, const void *__restrict__ wsrc)
-{
-    __shared__ float2 w[9 * COUT * CIN];
-    for (int i = threadIdx.x; i < 9 * COUT * CIN; i += blockDim.x) {
-        const int p = i / (COUT * CIN), a = (i / CIN) % COUT, b = i % CIN;
-        const int src = ADJ ? (rev_path(p) * CIN + b) * COUT + a : i;
+// Weights of a full-lattice layer CIN -> COUT as get(p, a, b): W[9][COUT][CIN],
+// or (ADJ) the adjoint of the layer W[9][CIN][COUT], A[p][a][b] = conj(W[rev
+// p][b][a]); FP32 or BF16 source.
+template <int CIN, int COUT, bool ADJ, bool BF> struct LayerWeights {
+    const void *w;
+    __device__ __forceinline__ float2 operator()(int p, int a, int b) const
+    {
+        const int i = ADJ ? (rev_path(p) * CIN + b) * COUT + a : (p * COUT + a) * CIN + b;
         float2 v;
         if (BF) {
-            const uint32_t h = ((const uint32_t *)wsrc)[src];
+            const uint32_t h = ((const uint32_t *)w)[i];
             v = make_float2(bf2f(h & 0xffffu), bf2f(h >> 16));
         } else {
-            v = ((const float2 *)wsrc)[src];
+            v = ((const float2 *)w)[i];
         }
         if (ADJ) v.y = -v.y;
-        w[i] = v;
+        return v;
     }
-    __syncthreads();
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= g.V) return;
-    const int V = g.V;
-    int x[4];
-    coords_of(g, s, x);
-    Cx<float> acc[COUT][3];
-#pragma unroll
-    for (int a = 0; a < COUT; a++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) acc[a][c] = {0.f, 0.f};
+};
 
-    for (int p = 0; p < 9; p++) {
-        const Hop h = path_hop(g, x, s, p);
-        Cx<float> u[9];
-        if (p > 0) load_link(U, h, p, u);
-        if (CIN <= COUT) {
-            // transport each input channel, then mix into all outputs
-#pragma unroll
-            for (int b = 0; b < CIN; b++) {
-                Cx<float> v[3], t[3];
-#pragma unroll
-                for (int c = 0; c < 3; c++) v[c] = ldf(in, b * 3 + c, V, h.sn);
-                if (p > 0) matvec(u, v, t);
-                else {
-#pragma unroll
-                    for (int c = 0; c < 3; c++) t[c] = v[c];
-                }
-#pragma unroll
-                for (int a = 0; a < COUT; a++) {
-                    const float2 wv = w[(p * COUT + a) * CIN + b];
-                    const Cx<float> wc{wv.x, wv.y};
-#pragma unroll
-                    for (int c = 0; c < 3; c++) acc[a][c] = acc[a][c] + cmul(wc, t[c]);
-                }
-            }
-        } else {
-            // mix the input channels at the neighbour, then transport COUT vectors
-            Cx<float> m[COUT][3];
-#pragma unroll
-            for (int a = 0; a < COUT; a++)
-#pragma unroll
-                for (int c = 0; c < 3; c++) m[a][c] = {0.f, 0.f};
-#pragma unroll
-            for (int b = 0; b < CIN; b++) {
-                Cx<float> v[3];
-#pragma unroll
-                for (int c = 0; c < 3; c++) v[c] = ldf(in, b * 3 + c, V, h.sn);
-#pragma unroll
-                for (int a = 0; a < COUT; a++) {
-                    const float2 wv = w[(p * COUT + a) * CIN + b];
-                    const Cx<float> wc{wv.x, wv.y};
-#pragma unroll
-                    for (int c = 0; c < 3; c++) m[a][c] = m[a][c] + cmul(wc, v[c]);
-                }
-            }
-#pragma unroll
-            for (int a = 0; a < COUT; a++) {
-                Cx<float> t[3];
-                if (p > 0) matvec(u, m[a], t);
-                else {
-#pragma unroll
-                    for (int c = 0; c < 3; c++) t[c] = m[a][c];
-                }
-#pragma unroll
-                for (int c = 0; c < 3; c++) acc[a][c] = acc[a][c] + t[c];
-            }
-        }
-    }
-#pragma unroll
-    for (int a = 0; a < COUT; a++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) out[(size_t)(a * 3 + c) * V + s] = make_float2(acc[a][c].re, acc[a][c].im);
+// The full-lattice layers run three wavefronts per 64 sites, each on three of
+// the nine paths, whose sums the first one adds up through LDS: at the
+// training lattice one wavefront per 64 sites would be two per SIMD, too few
+// to cover the gathers.  16^3x32, CH = 16: 4 -> 16 takes 38 us (48 us with the
+// mixing on the vector ALU), 16 -> 4 takes 48 us (76 us; 73 us with one
+// wavefront per 64 sites).
+constexpr int kLayerT = 192;
+// this thread's site (clamped to the lattice) and whether it is its own; w its wavefront
+__device__ __forceinline__ NetSite layer_site(const Geom &g, int nblk8, bool &own, int &w)
+{
+    w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int u = net_block(nblk8) * 64 + (int)(threadIdx.x & 63);
+    own = u < g.V;
+    const int s = min(u, g.V - 1);
+    const int p = s >= g.Vh ? 1 : 0;
+    return net_site(g, p, s - p * g.Vh);
 }
 
-// Weight gradient of a layer CIN -> COUT: G[p][a][b] = sum_x sum_c g_a(x)_c
-// conj((T_p in_b)(x)_c).  grid = (blocks over sites, 9 paths, 4x4 tiles of
-// (a, b)); per-workgroup partials, summed in a fixed order by wgrad_finish.
-template <int CIN, int COUT>
-__global__ __launch_bounds__(kT) void ptc_wgrad_kernel(const float2 *__restrict__ gin, const float2 *__restrict__ in,
-                                                       GaugeF18 U, Geom geo, double *__restrict__ part)
+// Full-lattice layer 4 -> CH (or the adjoint of a layer CH -> 4).
+template <int CH, bool ADJ, bool BF, class S>
+__global__ __launch_bounds__(kLayerT) QKX_NET_REGS void net_expand_kernel(S in, Hid out, GaugeF18 U, Geom g, int nblk8,
+                                                                          LayerWeights<4, CH, ADJ, BF> wt)
 {
-    const int p = blockIdx.y;
-    const int a0 = (blockIdx.z / (CIN / 4)) * 4, b0 = (blockIdx.z % (CIN / 4)) * 4;
-    const int V = geo.V;
-    float acc[4][4][2];
+    constexpr int H = CH / 4;
+    __shared__ f4v part[2][H * 6][64];
+    bool own;
+    int w;
+    const NetSite n = layer_site(g, nblk8, own, w);
+    f4v re[H][3], im[H][3];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j][0] = acc[i][j][1] = 0.f;
-    for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < V; s += gridDim.x * blockDim.x) {
-        int x[4];
-        coords_of(geo, s, x);
-        const Hop h = path_hop(geo, x, s, p);
-        Cx<float> u[9];
-        if (p > 0) load_link(U, h, p, u);
-        Cx<float> t[4][3];
-#pragma unroll
-        for (int bb = 0; bb < 4; bb++) {
-            Cx<float> v[3];
-#pragma unroll
-            for (int c = 0; c < 3; c++) v[c] = ldf(in, (b0 + bb) * 3 + c, V, h.sn);
-            if (p > 0) matvec(u, v, t[bb]);
-            else {
-#pragma unroll
-                for (int c = 0; c < 3; c++) t[bb][c] = v[c];
-            }
-        }
-#pragma unroll
-        for (int aa = 0; aa < 4; aa++) {
-            Cx<float> gv[3];
-#pragma unroll
-            for (int c = 0; c < 3; c++) gv[c] = ldf(gin, (a0 + aa) * 3 + c, V, s);
-#pragma unroll
-            for (int bb = 0; bb < 4; bb++) {
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    const Cx<float> z = cjmul(t[bb][c], gv[c]);   // g * conj(t)
-                    acc[aa][bb][0] += z.re;
-                    acc[aa][bb][1] += z.im;
-                }
-            }
-        }
+    for (int h = 0; h < H; h++) {
+        zero3(re[h]);
+        zero3(im[h]);
     }
-    // workgroup sum of the 32 values: wavefront butterflies, then LDS
-    __shared__ float red[kT / 64][32];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    auto unit = [](int site) { return site; };
+    const LinkGlobal ls{U, g, n};
+    if (w == 0) expand<CH, 0, 3>(in, ls, n, unit, wt, re, im);
+    else if (w == 1) expand<CH, 3, 6>(in, ls, n, unit, wt, re, im);
+    else expand<CH, 6, 9>(in, ls, n, unit, wt, re, im);
+    const int lane = threadIdx.x & 63;
+    if (w > 0) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+        for (int h = 0; h < H; h++)
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int k = 0; k < 2; k++) {
-                float v = acc[i][j][k];
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-                if (lane == 0) red[wv][(i * 4 + j) * 2 + k] = v;
+            for (int c = 0; c < 3; c++) {
+                part[w - 1][h * 6 + c][lane] = re[h][c];
+                part[w - 1][h * 6 + 3 + c][lane] = im[h][c];
             }
+    }
     __syncthreads();
-    if (threadIdx.x < 32) {
-        double s = 0;
-        for (int q = 0; q < (int)(blockDim.x >> 6); q++) s += red[q][threadIdx.x];
-        const int i = threadIdx.x >> 3, j = (threadIdx.x >> 1) & 3, k = threadIdx.x & 1;
-        const int widx = (p * COUT + a0 + i) * CIN + b0 + j;
-        part[((size_t)blockIdx.x * 9 * COUT * CIN + widx) * 2 + k] = s;
+    if (w > 0) return;
+#pragma unroll
+    for (int h = 0; h < H; h++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            re[h][c] += part[0][h * 6 + c][lane] + part[1][h * 6 + c][lane];
+            im[h][c] += part[0][h * 6 + 3 + c][lane] + part[1][h * 6 + 3 + c][lane];
+        }
+    if (own) {
+#pragma unroll
+        for (int h = 0; h < H; h++) out.store(h, n.s, re[h], im[h]);
     }
 }
 
-__global__ void wgrad_finish_kernel(const double *__restrict__ part, int nblocks, int nw, double2 *grad)
+// Full-lattice layer CH -> 4.  LOSS: the pair loss of the output o against
+// the target e instead: out = 2 (o - e), per-workgroup |o - e|^2.
+template <int CH, bool BF, bool LOSS, class S, class E>
+__global__ __launch_bounds__(kLayerT) QKX_NET_REGS void net_contract_kernel(Hid in, S out, E e, GaugeF18 U, Geom g,
+                                                                            int nblk8, LayerWeights<CH, 4, false, BF> wt,
+                                                                            double *lpart)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nw) return;
-    double re = 0, im = 0;
-    for (int b = 0; b < nblocks; b++) {
-        re += part[((size_t)b * nw + i) * 2];
-        im += part[((size_t)b * nw + i) * 2 + 1];
+    __shared__ float part[2][24][64];
+    bool own;
+    int w;
+    const NetSite n = layer_site(g, nblk8, own, w);
+    Cx<float> acc[12];
+#pragma unroll
+    for (int k = 0; k < 12; k++) acc[k] = {0.f, 0.f};
+    auto unit = [](int site) { return site; };
+    const LinkGlobal ls{U, g, n};
+    if (w == 0) contract<CH, 0, 3>(in, ls, n, unit, wt, acc);
+    else if (w == 1) contract<CH, 3, 6>(in, ls, n, unit, wt, acc);
+    else contract<CH, 6, 9>(in, ls, n, unit, wt, acc);
+    const int lane = threadIdx.x & 63;
+    if (w > 0) {
+#pragma unroll
+        for (int k = 0; k < 12; k++) {
+            part[w - 1][2 * k][lane] = acc[k].re;
+            part[w - 1][2 * k + 1][lane] = acc[k].im;
+        }
     }
-    grad[i].x += re;
-    grad[i].y += im;
+    __syncthreads();
+    if (w > 0) return;
+#pragma unroll
+    for (int k = 0; k < 12; k++) {
+        acc[k].re += part[0][2 * k][lane] + part[1][2 * k][lane];
+        acc[k].im += part[0][2 * k + 1][lane] + part[1][2 * k + 1][lane];
+    }
+    double d2 = 0;
+    if (own) {
+        if constexpr (LOSS) {
+            Cx<typename E::Real> t[12];
+            e.load(n.s, t);
+#pragma unroll
+            for (int k = 0; k < 12; k++) {
+                const float dx = acc[k].re - (float)t[k].re, dy = acc[k].im - (float)t[k].im;
+                acc[k] = {2.f * dx, 2.f * dy};
+                d2 += (double)dx * dx + (double)dy * dy;
+            }
+        }
+        Cx<typename S::Real> o[12];
+#pragma unroll
+        for (int k = 0; k < 12; k++) o[k] = {acc[k].re, acc[k].im};
+        out.store(n.s, o);
+    }
+    if constexpr (LOSS) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) d2 += __shfl_xor(d2, off, 64);
+        if (lane == 0) lpart[blockIdx.x] = d2;
+    }
 }
 
-// loss of one pair: d = o - e, gout = 2 d, per-workgroup |d|^2
-__global__ __launch_bounds__(kT) void loss_kernel(const float2 *__restrict__ o, const float2 *__restrict__ e,
-                                                  float2 *__restrict__ gout, int n, double *part)
+// ---------------------------------------------------------------------------
+// Weight gradients of both layers in one form: for a CH-channel field f and a
+// 4-channel field v,
+//   Z[p][j][k] = sum_y sum_c f_k(y)_c conj((T_p v_j)(y)_c).
+// Layer 1 (f = gh, v = r): dL/dW1[p][a][b] = Z[p][b][a].  Layer 2 (f = h, v =
+// gout): a sum over all sites may be taken at the other end of the path, and
+// T_p and T_rev(p) are adjoint, so dL/dW2[p][a][b] = conj(Z[rev p][a][b]).
+//
+// The sum over sites is a contraction on the matrix cores: v_mfma_f32_4x4x1
+// adds the 4 x 4 outer product of four lanes' real numbers (rows: channels 4 h
+// + i of f, columns: vectors i of T_p v, one site) to each of its 16 blocks'
+// own sums.  Lane = site for the loads and transports, so that a load reads
+// consecutive sites (16 cache accesses; with the four channels of a site on
+// adjacent lanes every lane was an access of its own) and a link is fetched
+// once per site; a 4 x 4 transposition within each quad of lanes (8 selects
+// with a lane-permuted source per 4 registers) then turns four sites' numbers
+// into four rounds of MFMA operands.  blockIdx.y is a group of NP paths; the
+// sums stay in registers over the sites.  16^3x32, CH = 16: 70 us a layer
+// (125 us on the vector ALU, where f and v were read once per path), bound by
+// the gathers' latency at two wavefronts per SIMD; the whole gradient of a pair,
+// tm included, 592 -> 306 us.
+// Partials: part[(widx * 2 + re/im) * gridDim.x + blockIdx.x] with widx = (p *
+// 4 + j) * CH + k, summed in a fixed order.
+__device__ __forceinline__ float row_sum(float v)   // sum over lanes of equal l % 4 in 16 lanes
 {
-    double acc = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const float2 a = o[i], b = e[i];
-        const float dx = a.x - b.x, dy = a.y - b.y;
-        gout[i] = make_float2(2.f * dx, 2.f * dy);
-        acc += (double)dx * dx + (double)dy * dy;
-    }
-    __shared__ double red[kT / 64];
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, true));   // row_ror:4
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));   // row_ror:8
+    return v;
+}
+// a[i] of lane j <-> a[j] of lane i within each quad of lanes
+template <int CTRL> __device__ __forceinline__ void quad_swap(float &x, float &y, bool upper)
+{
+    const float px = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+    const float py = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(y), CTRL, 0xf, 0xf, true));
+    x = upper ? py : x;
+    y = upper ? y : px;
+}
+__device__ __forceinline__ void quad_transpose(float &a, float &b, float &c, float &d)
+{
+    const bool u1 = threadIdx.x & 1, u2 = threadIdx.x & 2;
+    quad_swap<0xB1>(a, b, u1);   // lanes 1 0 3 2
+    quad_swap<0xB1>(c, d, u1);
+    quad_swap<0x4E>(a, c, u2);   // lanes 2 3 0 1
+    quad_swap<0x4E>(b, d, u2);
+}
+// four colour vectors of the lane's site -> v[3 r + c]: the lane's vector (lane
+// & 3) of the quad's site r; zero for lanes past the end
+__device__ __forceinline__ void quad_vectors(Cx<float> v[12], bool live)
+{
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    for (int k = 0; k < 12; k++)
+        if (!live) v[k] = {0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        quad_transpose(v[c].re, v[3 + c].re, v[6 + c].re, v[9 + c].re);
+        quad_transpose(v[c].im, v[3 + c].im, v[6 + c].im, v[9 + c].im);
+    }
+}
+// the operands of one path
+template <class S> struct GradOps {
+    typename S::Raw psi;
+    GaugeF18::Raw link;
+};
+template <int P, class S>
+__device__ __forceinline__ void wgrad_fetch(const S &v, const GaugeF18 &U, const Geom &g, const NetSite &n, GradOps<S> &o)
+{
+    o.psi = v.template fetch<3>(path_site<P>(n));
+    if constexpr (P > 0) o.link = LinkGlobal{U, g, n}.template fetch<P>();
+}
+// t = T_P v of the lane's site, as quad_vectors leaves it
+template <int P, class S>
+__device__ __forceinline__ void wgrad_transport(const S &v, const GaugeF18 &U, const Geom &g, const NetSite &n, bool live,
+                                                const GradOps<S> &o, Cx<float> t[12])
+{
+    Cx<float> x[12];
+    (void)unpack_spinor(v, o.psi, x);
+    if constexpr (P == 0) {
+#pragma unroll
+        for (int k = 0; k < 12; k++) t[k] = x[k];
+    } else {
+        Cx<float> l[9];
+        LinkGlobal{U, g, n}.template get<P, false>(o.link, 1.0f, l);
+#pragma unroll
+        for (int b = 0; b < 4; b++) transport<P>(l, x + 3 * b, t + 3 * b);
+    }
+    quad_vectors(t, live);
+}
+// no later load is issued before this point: the fetches stay one step ahead
+__device__ __forceinline__ void wgrad_step() { asm volatile("" ::: "memory"); }
+// z[q] += f conj(t[q]) over the quad's four sites, the NP sums interleaved so
+// that no MFMA waits for the one before it
+template <int NP>
+__device__ __forceinline__ void wgrad_tiles(const Cx<float> f[12], const Cx<float> (*t)[12], f4v *zr, f4v *zi, int stride)
+{
+#pragma unroll
+    for (int k = 0; k < 12; k++) {
+#pragma unroll
+        for (int q = 0; q < NP; q++) zr[q * stride] = __builtin_amdgcn_mfma_f32_4x4x1f32(f[k].re, t[q][k].re, zr[q * stride], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < NP; q++) zi[q * stride] = __builtin_amdgcn_mfma_f32_4x4x1f32(f[k].im, t[q][k].re, zi[q * stride], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < NP; q++) zr[q * stride] = __builtin_amdgcn_mfma_f32_4x4x1f32(f[k].im, t[q][k].im, zr[q * stride], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < NP; q++) zi[q * stride] = __builtin_amdgcn_mfma_f32_4x4x1f32(f[k].re, -t[q][k].im, zi[q * stride], 0, 0, 0);
+    }
+}
+// one tile per path (CH = 4): f stays, the transports come one at a time
+template <int P, int P1, class S>
+__device__ __forceinline__ void wgrad_each(const S &v, const GaugeF18 &U, const Geom &g, const NetSite &n, bool live,
+                                           const GradOps<S> &o, const Cx<float> f[12], f4v (*zr)[1], f4v (*zi)[1])
+{
+    GradOps<S> next;
+    if constexpr (P + 1 < P1) wgrad_fetch<P + 1>(v, U, g, n, next);
+    Cx<float> t[1][12];
+    wgrad_transport<P>(v, U, g, n, live, o, t[0]);
+    wgrad_tiles<1>(f, t, zr[0], zi[0], 1);
+    wgrad_step();
+    if constexpr (P + 1 < P1) wgrad_each<P + 1, P1>(v, U, g, n, live, next, f, zr + 1, zi + 1);
+}
+// the transports of paths P .. P1 - 1, and f's first channels requested
+template <int P, int P1, class S>
+__device__ __forceinline__ void wgrad_hold(const S &v, const GaugeF18 &U, const Geom &g, const NetSite &n, bool live,
+                                           const GradOps<S> &o, Cx<float> (*t)[12], const Hid &f, Hid::Raw &fr)
+{
+    GradOps<S> next;
+    if constexpr (P + 1 < P1) wgrad_fetch<P + 1>(v, U, g, n, next);
+    else fr = f.fetch(0, n.s);
+    wgrad_transport<P>(v, U, g, n, live, o, *t);
+    wgrad_step();
+    if constexpr (P + 1 < P1) wgrad_hold<P + 1, P1>(v, U, g, n, live, next, t + 1, f, fr);
+}
+template <int CH, int P0, int NP, class S>
+__device__ __forceinline__ void wgrad_group(const Hid &f, const S &v, const GaugeF18 &U, const Geom &g, double *part)
+{
+    constexpr int H = CH / 4;
+    f4v zr[NP][H], zi[NP][H];
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+        for (int h = 0; h < H; h++) zr[p][h] = zi[p][h] = f4v{0.f, 0.f, 0.f, 0.f};
+    const int i = threadIdx.x & 3;
+    // the same number of rounds in every wavefront of the workgroup
+    for (int s0 = blockIdx.x * blockDim.x; s0 < g.V; s0 += gridDim.x * blockDim.x) {
+        const int s1 = s0 + (int)threadIdx.x;
+        const bool live = s1 < g.V;
+        const int s = min(s1, g.V - 1);
+        const int p = s >= g.Vh ? 1 : 0;
+        const NetSite n = net_site(g, p, s - p * g.Vh);
+        Cx<float> ff[12];
+        GradOps<S> o0;
+        wgrad_fetch<P0>(v, U, g, n, o0);
+        if constexpr (H == 1) {
+            Hid::unpack(f.fetch(0, s), ff);
+            quad_vectors(ff, live);
+            wgrad_each<P0, P0 + NP>(v, U, g, n, live, o0, ff, zr, zi);
+        } else {   // the transports stay, the channels come four at a time
+            Cx<float> t[NP][12];
+            Hid::Raw fr;
+            wgrad_hold<P0, P0 + NP>(v, U, g, n, live, o0, t, f, fr);
+#pragma unroll
+            for (int h = 0; h < H; h++) {
+                Hid::unpack(fr, ff);
+                if (h + 1 < H) fr = f.fetch(h + 1, s);
+                quad_vectors(ff, live);
+                wgrad_tiles<NP>(ff, t, &zr[0][h], &zi[0][h], H);
+                wgrad_step();
+            }
+        }
+    }
+    // sums of 16 lanes' blocks in registers, of the workgroup's 16-lane rows in LDS and FP64
+    __shared__ float red[NP * H * 8 * 4][kT / 16 + 1];
+    const int row = threadIdx.x >> 4, rows = blockDim.x >> 4;
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+        for (int h = 0; h < H; h++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                zr[p][h][k] = row_sum(zr[p][h][k]);
+                zi[p][h][k] = row_sum(zi[p][h][k]);
+            }
+    if ((threadIdx.x & 12) == 0) {
+#pragma unroll
+        for (int p = 0; p < NP; p++)
+#pragma unroll
+            for (int h = 0; h < H; h++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const int w = (p * 4 + i) * CH + 4 * h + k;   // row k: channel of f, column i: vector of v
+                    red[2 * w][row] = zr[p][h][k];
+                    red[2 * w + 1][row] = zi[p][h][k];
+                }
+    }
     __syncthreads();
+    for (int w = threadIdx.x; w < NP * 4 * CH * 2; w += blockDim.x) {
+        double t = 0;
+        for (int q = 0; q < rows; q++) t += (double)red[w][q];
+        part[(size_t)(P0 * 4 * CH * 2 + w) * gridDim.x + blockIdx.x] = t;
+    }
+}
+// paths per group: the sums take 2 CH registers per path, the transports held
+// beside them 24; one more path per group spills (CH = 16: 83 us with three)
+constexpr int wgrad_np(int ch) { return ch == 4 ? 9 : ch == 8 ? 3 : 2; }
+constexpr int wgrad_groups(int ch) { return (9 + wgrad_np(ch) - 1) / wgrad_np(ch); }
+template <int CH, int G, class S>
+__device__ __forceinline__ void wgrad_select(const Hid &f, const S &v, const GaugeF18 &U, const Geom &g, double *part)
+{
+    constexpr int P0 = G * wgrad_np(CH), NP = P0 + wgrad_np(CH) <= 9 ? wgrad_np(CH) : 9 - P0;
+    if constexpr (G + 1 == wgrad_groups(CH)) wgrad_group<CH, P0, NP>(f, v, U, g, part);
+    else if ((int)blockIdx.y == G) wgrad_group<CH, P0, NP>(f, v, U, g, part);
+    else wgrad_select<CH, G + 1>(f, v, U, g, part);
+}
+template <int CH, class S>
+__global__ __launch_bounds__(kT) QKX_NET_REGS void net_wgrad_kernel(Hid f, S v, GaugeF18 U, Geom g, double *part)
+{
+    wgrad_select<CH, 0>(f, v, U, g, part);
+}
+
+// The gradient of both layers and the loss from their partials, one wavefront
+// per number: workgroup w < nw is complex weight w of layer 1, then of layer
+// 2, the last one the loss.
+__global__ __launch_bounds__(64) void grad_finish_kernel(const double *z1, const double *z2, int nb, const double *lpart,
+                                                         int nl, int ch, double2 *grad, double *loss)
+{
+    const int w = blockIdx.x, n1 = 9 * 4 * ch;
+    auto sum = [&](const double *p, int n) {
+        double t = 0;
+        for (int i = threadIdx.x; i < n; i += 64) t += p[i];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+        return t;
+    };
+    if (w == 2 * n1) {
+        const double t = sum(lpart, nl);
+        if (threadIdx.x == 0) *loss += t;
+        return;
+    }
+    const bool first = w < n1;
+    const int i = first ? w : w - n1;
+    // weight [p][a][b]: layer 1 [9][ch][4] takes Z[p][b][a], layer 2 [9][4][ch] conj(Z[rev p][a][b])
+    const int p = i / (4 * ch), r = i % (4 * ch);
+    const int zi = first ? (p * 4 + r % 4) * ch + r / 4 : (rev_path(p) * 4 + r / ch) * ch + r % ch;
+    const double *z = first ? z1 : z2;
+    const double re = sum(z + (size_t)(2 * zi) * nb, nb), im = sum(z + (size_t)(2 * zi + 1) * nb, nb);
     if (threadIdx.x == 0) {
-        double s = 0;
-        for (int q = 0; q < (int)(blockDim.x >> 6); q++) s += red[q];
-        part[blockIdx.x] = s;
+        grad[w].x += re;
+        grad[w].y += first ? im : -im;
     }
-}
-
-__global__ void loss_finish_kernel(const double *part, int nblocks, double *loss)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double s = 0;
-    for (int b = 0; b < nblocks; b++) s += part[b];
-    *loss += s;
 }
 
 __global__ void adam_kernel(float2 *w, uint32_t *wb, double2 *grad, float2 *m, float2 *v, int n, float lr,
@@ -375,300 +440,52 @@ __global__ void to_bf16_kernel(const float2 *w, uint32_t *wb, int n)
     if (i < n) wb[i] = f2bf(w[i].x) | (f2bf(w[i].y) << 16);
 }
 
-// spinor field (accessor S, full lattice) <-> 4-channel feature field
-template <class S> __global__ __launch_bounds__(kT) void spinor_to_feat(S f, float2 *out, int V)
+int layer_blocks(int V) { return (V + 63) / 64; }
+// workgroups of a layer launch after XCD remapping: one loss partial each
+int loss_blocks(int V)
 {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= V) return;
-    Cx<typename S::Real> v[12];
-    f.load(s, v);
-#pragma unroll
-    for (int k = 0; k < 12; k++) out[(size_t)k * V + s] = make_float2((float)v[k].re, (float)v[k].im);
+    int nb = layer_blocks(V);
+    (void)net_remap(nb);
+    return nb;
 }
-template <class S> __global__ __launch_bounds__(kT) void feat_to_spinor(const float2 *in, S f, int V)
+// workgroup size and count of the weight gradient
+// (of each path group): as many as are resident at two wavefronts per SIMD,
+// all with the same number of rounds, so that the sums' way through LDS and
+// memory is paid once per resident workgroup
+constexpr int kGradBlocks = 512;
+void grad_grid(int ch, int V, int &bs, int &nb)
 {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= V) return;
-    using R = typename S::Real;
-    Cx<R> v[12];
-#pragma unroll
-    for (int k = 0; k < 12; k++) {
-        const float2 a = in[(size_t)k * V + s];
-        v[k] = {(R)a.x, (R)a.y};
-    }
-    f.store(s, v);
+    const int groups = wgrad_groups(ch);
+    bs = V >= kGradBlocks / groups * kT ? kT : 64;
+    const int most = kGradBlocks * (kT / bs) / groups, tiles = (V + bs - 1) / bs;
+    const int rounds = (tiles + most - 1) / most;
+    nb = (tiles + rounds - 1) / rounds;
 }
-
-// ---------------------------------------------------------------------------
-// The network on even-parity fields, N_e = P_e L2 L1 P_e (P_e: restriction to
-// the even sites), batched over right-hand sides (RHS innermost).  With the
-// input zero on the odd sites, L1's hidden channels are W1[0] in(x) at an even
-// site x and sum_{p>0} W1[p] (T_p in)(y) at an odd site y (all neighbours of y
-// are even), and L2's output at x is
-//   C0 in(x) + sum_{p>0} W2[p] (T_p h)(x),   C0 = W2[0] W1[0]  (4 x 4),
-// whose hops read only odd-site hidden channels.  So N_e is two launches:
-// eo_hidden_kernel (odd sites) and eo_out_kernel (even sites).  The adjoint
-// N_e^dag = P_e L1^dag L2^dag P_e has the same form with the adjoint layers'
-// weights, A[p][a][b] = conj(W[rev p][b][a]).
-//
-// Weight table of one direction (forward or adjoint), complex:
-//   [8][CH][4] first-layer hops (p = 1..8), [8][4][CH] second-layer hops,
-//   [4][4] C0.
-constexpr int eo_table(int ch) { return 8 * ch * 4 * 2 + 16; }
-
-__device__ __forceinline__ float2 net_w(const float2 *w, const uint32_t *wb, int bf, int i)
-{
-    if (!bf) return w[i];
-    const uint32_t h = wb[i];
-    return make_float2(bf2f(h & 0xffffu), bf2f(h >> 16));
-}
-
-// Both tables from the FP32 master weights or their BF16 copies: thread i
-// writes entry i of [forward table][adjoint table].
-__global__ void eo_weights_kernel(const float2 *w, const uint32_t *wb, int bf, int ch, float2 *out)
-{
-    const int T = eo_table(ch), i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 2 * T) return;
-    const int adj = i / T, j = i % T, n1 = 9 * ch * 4;
-    auto W1 = [&](int p, int a, int b) { return net_w(w, wb, bf, (p * ch + a) * 4 + b); };    // [9][ch][4]
-    auto W2 = [&](int p, int a, int b) { return net_w(w, wb, bf, n1 + (p * 4 + a) * ch + b); };   // [9][4][ch]
-    auto cj = [](float2 v) { return make_float2(v.x, -v.y); };
-    const int h1 = 8 * ch * 4;
-    float2 v;
-    if (j < h1) {                       // first layer, p = 1..8: [a < ch][b < 4]
-        const int p = j / (ch * 4) + 1, a = (j / 4) % ch, b = j % 4;
-        v = adj ? cj(W2(rev_path(p), b, a)) : W1(p, a, b);
-    } else if (j < 2 * h1) {            // second layer: [a < 4][b < ch]
-        const int k = j - h1, p = k / (4 * ch) + 1, a = (k / ch) % 4, b = k % ch;
-        v = adj ? cj(W1(rev_path(p), b, a)) : W2(p, a, b);
-    } else {                            // C0 = W2[0] W1[0], or its adjoint
-        const int k = j - 2 * h1, a = adj ? k % 4 : k / 4, b = adj ? k / 4 : k % 4;
-        float re = 0.f, im = 0.f;
-        for (int c = 0; c < ch; c++) {
-            const float2 x = W2(0, a, c), y = W1(0, c, b);
-            re += x.x * y.x - x.y * y.y;
-            im += x.x * y.y + x.y * y.x;
-        }
-        v = adj ? make_float2(re, -im) : make_float2(re, im);
-    }
-    out[i] = v;
-}
-
-// Hidden channels at the odd sites: h_a(y) = sum_{p>0} sum_b w[p][a][b] (T_p in_b)(y).
-// One thread per (odd site, RHS); in is an even-parity field.
-template <int CH, class S>
-__global__ __launch_bounds__(kT) void eo_hidden_kernel(S in, GaugeF18 U, Geom g, const float2 *__restrict__ wsrc,
-                                                       float2 *__restrict__ hid, int nr, int r0, int nc,
-                                                       const int *skip)
-{
-    if (skip && *skip) return;   // uniform over the grid
-    __shared__ float2 w[8 * CH * 4];
-    for (int i = threadIdx.x; i < 8 * CH * 4; i += blockDim.x) w[i] = wsrc[i];
-    __syncthreads();
-    // units of this launch: (odd site, rhs r0 .. r0 + nc - 1) of a batch of nr
-    const int u = blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= g.Vh * nc) return;
-    const int cb = u / nc, r = r0 + (u - cb * nc);
-    const int s = g.Vh + cb;
-    int x[4];
-    coords_of(g, s, x);
-    Cx<float> acc[CH][3];
-#pragma unroll
-    for (int a = 0; a < CH; a++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) acc[a][c] = {0.f, 0.f};
-    for (int p = 1; p < 9; p++) {
-        const Hop h = path_hop(g, x, s, p);   // h.sn: an even site, = its checkerboard index
-        Cx<float> uu[9];
-        load_link(U, h, p, uu);
-        Cx<typename S::Real> v[12];
-        in.load(h.sn * nr + r, v);
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const Cx<float> vb[3] = {{(float)v[b * 3].re, (float)v[b * 3].im},
-                                     {(float)v[b * 3 + 1].re, (float)v[b * 3 + 1].im},
-                                     {(float)v[b * 3 + 2].re, (float)v[b * 3 + 2].im}};
-            Cx<float> t[3];
-            matvec(uu, vb, t);
-#pragma unroll
-            for (int a = 0; a < CH; a++) {
-                const float2 wv = w[((p - 1) * CH + a) * 4 + b];
-                const Cx<float> wc{wv.x, wv.y};
-#pragma unroll
-                for (int c = 0; c < 3; c++) acc[a][c] = acc[a][c] + cmul(wc, t[c]);
-            }
-        }
-    }
-    const size_t stride = (size_t)g.Vh * nc;
-#pragma unroll
-    for (int a = 0; a < CH; a++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) hid[(size_t)(a * 3 + c) * stride + u] = make_float2(acc[a][c].re, acc[a][c].im);
-}
-
-// Output at the even sites: out(x) = C0 in(x) + sum_{p>0} (T_p m_p)(x) with
-// m_p = w[p] h at the odd neighbour (the channels are mixed first, then the
-// four colour vectors transported).  One thread per (even site, RHS).
-template <int CH, class S>
-__global__ __launch_bounds__(kT) void eo_out_kernel(S in, S out, GaugeF18 U, Geom g, const float2 *__restrict__ wsrc,
-                                                    const float2 *__restrict__ hid, int nr, int r0, int nc,
-                                                    const int *skip)
-{
-    if (skip && *skip) return;   // uniform over the grid
-    __shared__ float2 w[8 * 4 * CH + 16];
-    for (int i = threadIdx.x; i < 8 * 4 * CH + 16; i += blockDim.x) w[i] = wsrc[i];
-    __syncthreads();
-    const int u = blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= g.Vh * nc) return;
-    const int cb = u / nc, rc = u - cb * nc;
-    const int e = cb * nr + r0 + rc;   // the unit's entry in the batch fields
-    int x[4];
-    coords_of(g, cb, x);
-    Cx<float> acc[4][3];
-    {
-        Cx<typename S::Real> v[12];
-        in.load(e, v);
-#pragma unroll
-        for (int a = 0; a < 4; a++)
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                Cx<float> z{0.f, 0.f};
-#pragma unroll
-                for (int b = 0; b < 4; b++) {
-                    const float2 wv = w[8 * 4 * CH + a * 4 + b];
-                    z = z + cmul(Cx<float>{wv.x, wv.y}, Cx<float>{(float)v[b * 3 + c].re, (float)v[b * 3 + c].im});
-                }
-                acc[a][c] = z;
-            }
-    }
-    const size_t stride = (size_t)g.Vh * nc;
-    for (int p = 1; p < 9; p++) {
-        const Hop h = path_hop(g, x, cb, p);   // h.sn: an odd site
-        const size_t hu = (size_t)(h.sn - g.Vh) * nc + rc;
-        Cx<float> m[4][3];
-#pragma unroll
-        for (int a = 0; a < 4; a++)
-#pragma unroll
-            for (int c = 0; c < 3; c++) m[a][c] = {0.f, 0.f};
-#pragma unroll
-        for (int k = 0; k < CH; k++) {
-            Cx<float> hv[3];
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const float2 t = hid[(size_t)(k * 3 + c) * stride + hu];
-                hv[c] = {t.x, t.y};
-            }
-#pragma unroll
-            for (int a = 0; a < 4; a++) {
-                const float2 wv = w[((p - 1) * 4 + a) * CH + k];
-                const Cx<float> wc{wv.x, wv.y};
-#pragma unroll
-                for (int c = 0; c < 3; c++) m[a][c] = m[a][c] + cmul(wc, hv[c]);
-            }
-        }
-        Cx<float> uu[9];
-        load_link(U, h, p, uu);
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-            Cx<float> t[3];
-            matvec(uu, m[a], t);
-#pragma unroll
-            for (int c = 0; c < 3; c++) acc[a][c] = acc[a][c] + t[c];
-        }
-    }
-    using R = typename S::Real;
-    Cx<R> o[12];
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) o[a * 3 + c] = {(R)acc[a][c].re, (R)acc[a][c].im};
-    out.store(e, o);
-}
-
-int nblk(int n) { return (n + kT - 1) / kT; }
 
 int net_buffers(qkx_net_s *n, const int L[4])
 {
-    if (n->fin && n->L[0] == L[0] && n->L[1] == L[1] && n->L[2] == L[2] && n->L[3] == L[3]) return QKX_SUCCESS;
-    float2 **bufs[5] = {&n->fin, &n->fh, &n->fout, &n->gout, &n->gh};
+    if (n->fh && n->L[0] == L[0] && n->L[1] == L[1] && n->L[2] == L[2] && n->L[3] == L[3]) return QKX_SUCCESS;
+    float4 **bufs[3] = {&n->fh, &n->gout, &n->gh};
     for (auto b : bufs) {
         if (*b) (void)hipFree(*b);
         *b = nullptr;
     }
     const size_t V = (size_t)L[0] * L[1] * L[2] * L[3];
-    const int chans[5] = {4, n->ch, 4, 4, n->ch};
-    for (int i = 0; i < 5; i++) QKX_HIP(hipMalloc(bufs[i], sizeof(float2) * 3 * chans[i] * V));
+    const int chans[3] = {n->ch, 4, n->ch};
+    for (int i = 0; i < 3; i++) QKX_HIP(hipMalloc(bufs[i], sizeof(float2) * 3 * chans[i] * V));
     for (int d = 0; d < 4; d++) n->L[d] = L[d];
-    const int need = (int)(nblk((int)V) * 9 * 4 * n->ch * 2 + 1024);
+    // partials: both layers' gradients, then the loss
+    int bs, nb;
+    grad_grid(n->ch, (int)V, bs, nb);
+    const size_t need = (size_t)nb * 2 * 9 * 4 * n->ch * 2 + loss_blocks((int)V);
     if (need > n->part_cap) {
         if (n->part) (void)hipFree(n->part);
         n->part = nullptr;
+        n->part_cap = 0;
         QKX_HIP(hipMalloc(&n->part, sizeof(double) * need));
         n->part_cap = need;
     }
     return QKX_SUCCESS;
-}
-
-int check_net_gauge(const qkx_gauge_s *U)
-{
-    if (U->prec != QKX_PREC_SINGLE || U->recon != QKX_RECON_18) {
-        qkx::set_error("net: the gauge field must be FP32 with 18 reals");
-        return QKX_ERR_ARG;
-    }
-    return QKX_SUCCESS;
-}
-
-template <int CIN, int COUT, bool ADJ>
-int launch_ptc(const float2 *in, float2 *out, const qkx_gauge_s *U, const void *w, bool bf)
-{
-    Geom g = qkx::make_geom(U->L, U->bc);
-    GaugeF18 G = make_gauge<GaugeF18>(U);
-    if (bf)
-        hipLaunchKernelGGL((ptc_kernel<CIN, COUT, ADJ, true>), dim3(nblk(g.V)), dim3(kT), 0, qkx::g_stream, in, out,
-                           G, g, w);
-    else
-        hipLaunchKernelGGL((ptc_kernel<CIN, COUT, ADJ, false>), dim3(nblk(g.V)), dim3(kT), 0, qkx::g_stream, in, out,
-                           G, g, w);
-    QKX_HIP(hipGetLastError());
-    return QKX_SUCCESS;
-}
-
-// forward of both layers from n->fin into n->fh and n->fout
-int net_forward(qkx_net_s *n, const qkx_gauge_s *U)
-{
-    const bool bf = n->bf16 != 0;
-    const void *w1 = bf ? (const void *)n->wb : (const void *)n->w;
-    const void *w2 = bf ? (const void *)(n->wb + n->n1) : (const void *)(n->w + n->n1);
-    int rc;
-    if (n->ch == 16) {
-        if ((rc = launch_ptc<4, 16, false>(n->fin, n->fh, U, w1, bf))) return rc;
-        return launch_ptc<16, 4, false>(n->fh, n->fout, U, w2, bf);
-    }
-    if (n->ch == 4) {
-        if ((rc = launch_ptc<4, 4, false>(n->fin, n->fh, U, w1, bf))) return rc;
-        return launch_ptc<4, 4, false>(n->fh, n->fout, U, w2, bf);
-    }
-    if ((rc = launch_ptc<4, 8, false>(n->fin, n->fh, U, w1, bf))) return rc;
-    return launch_ptc<8, 4, false>(n->fh, n->fout, U, w2, bf);
-}
-
-template <int CIN, int COUT>
-int launch_wgrad(const float2 *g, const float2 *in, const qkx_gauge_s *U, qkx_net_s *n, double2 *grad)
-{
-    Geom geo = qkx::make_geom(U->L, U->bc);
-    const int nbx = std::min(nblk(geo.V), 128);
-    hipLaunchKernelGGL((ptc_wgrad_kernel<CIN, COUT>), dim3(nbx, 9, (COUT / 4) * (CIN / 4)), dim3(kT), 0,
-                       qkx::g_stream, g, in, make_gauge<GaugeF18>(U), geo, n->part);
-    const int nw = 9 * COUT * CIN;
-    hipLaunchKernelGGL(wgrad_finish_kernel, dim3((nw + 255) / 256), dim3(256), 0, qkx::g_stream, n->part, nbx, nw,
-                       grad);
-    QKX_HIP(hipGetLastError());
-    return QKX_SUCCESS;
-}
-
-template <class F> int with_spinor(const qkx_spinor_s *f, F fn)
-{
-    return dispatch_prec(f->prec, [&](auto tag) { return fn(make_spinor<decltype(tag)>(f)); });
 }
 
 int check_spinor(const qkx_spinor_s *f, const qkx_gauge_s *U)
@@ -681,67 +498,92 @@ int check_spinor(const qkx_spinor_s *f, const qkx_gauge_s *U)
     return QKX_SUCCESS;
 }
 
-int to_feat(const qkx_spinor_s *f, float2 *out)
+// fn(accessor) for a full-lattice FP64 or FP32 spinor (check_spinor passed)
+template <class F> int with_spinor(const qkx_spinor_s *f, F fn)
 {
-    const int V = f->V;
-    return with_spinor(f, [&](auto S) {
-        if constexpr (std::is_same_v<decltype(S), SpinorD> || std::is_same_v<decltype(S), SpinorF>) {
-            hipLaunchKernelGGL((spinor_to_feat<decltype(S)>), dim3(nblk(V)), dim3(kT), 0, qkx::g_stream, S, out, V);
-            QKX_HIP(hipGetLastError());
-            return QKX_SUCCESS;
-        } else {
-            qkx::set_error("net: FP64/FP32 fields only");
-            return QKX_ERR_ARG;
-        }
-    });
+    if (f->prec == QKX_PREC_DOUBLE) return fn(make_spinor<SpinorD>(f));
+    return fn(make_spinor<SpinorF>(f));
 }
-
-int from_feat(const float2 *in, qkx_spinor_s *f)
+template <class F> int with_bf(const qkx_net_s *n, F fn)
 {
-    const int V = f->V;
-    return with_spinor(f, [&](auto S) {
-        if constexpr (std::is_same_v<decltype(S), SpinorD> || std::is_same_v<decltype(S), SpinorF>) {
-            hipLaunchKernelGGL((feat_to_spinor<decltype(S)>), dim3(nblk(V)), dim3(kT), 0, qkx::g_stream, in, S, V);
-            QKX_HIP(hipGetLastError());
-            return QKX_SUCCESS;
-        } else {
-            qkx::set_error("net: FP64/FP32 fields only");
-            return QKX_ERR_ARG;
-        }
-    });
+    if (n->bf16) return fn(std::true_type{});
+    return fn(std::false_type{});
 }
+Hid hid_of(float4 *p, int V) { return Hid{p, (size_t)V}; }
 
-// right-hand sides per launch of the even-odd network: all of them while
-// their hidden channels fit the bound (default kEoHiddenCap float2 entries,
-// 4 GiB), else fewer
-constexpr size_t kEoHiddenCap = size_t(1) << 29;
-int eo_chunk(const qkx_net_s *n, const qkx_spinor_s *in)
-{
-    const size_t per_rhs = (size_t)n->ch * 3 * (size_t)in->Vh;
-    const size_t cap = n->ehid_limit ? n->ehid_limit : kEoHiddenCap;
-    return (int)std::max<size_t>(1, std::min<size_t>((size_t)in->nrhs, cap / per_rhs));
-}
-
-template <int CH, class S>
-int launch_eo(qkx_net_s *n, qkx_spinor_s *out, const qkx_spinor_s *in, const qkx_gauge_s *U, int adjoint,
-              const int *skip)
+// layer 1 of a spinor, or (ADJ) the adjoint of layer 2, into a hidden field
+template <bool ADJ> int launch_expand(qkx_net_s *n, const qkx_spinor_s *in, const SpinorF *inf, Hid out, const qkx_gauge_s *U)
 {
     const Geom g = qkx::make_geom(U->L, U->bc);
-    const int nr = in->nrhs, nc = eo_chunk(n, in);
     const GaugeF18 G = make_gauge<GaugeF18>(U);
-    const float2 *tab = n->weo + (adjoint ? eo_table(CH) : 0);
-    // the right-hand sides in chunks of nc, so that the hidden channels of a
-    // chunk fit the buffer (out may be in: each chunk reads only its own
-    // columns before writing them)
-    for (int r0 = 0; r0 < nr; r0 += nc) {
-        const int c = std::min(nc, nr - r0), units = g.Vh * c;
-        hipLaunchKernelGGL((eo_hidden_kernel<CH, S>), dim3(nblk(units)), dim3(kT), 0, qkx::g_stream,
-                           make_spinor<S>(in), G, g, tab, n->ehid, nr, r0, c, skip);
-        hipLaunchKernelGGL((eo_out_kernel<CH, S>), dim3(nblk(units)), dim3(kT), 0, qkx::g_stream, make_spinor<S>(in),
-                           make_spinor<S>(out), G, g, tab + 8 * CH * 4, (const float2 *)n->ehid, nr, r0, c, skip);
-    }
-    QKX_HIP(hipGetLastError());
-    return QKX_SUCCESS;
+    int nb = layer_blocks(g.V);
+    const int nblk8 = net_remap(nb);
+    const int off = ADJ ? n->n1 : 0;
+    return with_ch(n, [&](auto CHC) {
+        constexpr int CH = decltype(CHC)::value;
+        return with_bf(n, [&](auto BFC) {
+            constexpr bool BF = decltype(BFC)::value;
+            const LayerWeights<4, CH, ADJ, BF> w{BF ? (const void *)(n->wb + off) : (const void *)(n->w + off)};
+            auto go = [&](auto S) {
+                hipLaunchKernelGGL((net_expand_kernel<CH, ADJ, BF, decltype(S)>), dim3(nb), dim3(kLayerT), 0,
+                                   qkx::g_stream, S, out, G, g, nblk8, w);
+                QKX_HIP(hipGetLastError());
+                return QKX_SUCCESS;
+            };
+            if constexpr (ADJ) return go(*inf);
+            else return with_spinor(in, go);
+        });
+    });
+}
+
+// layer 2 into a spinor, or (e given) the loss gradient 2 (o - e) into gout
+// and per-workgroup losses into lpart
+int launch_contract(qkx_net_s *n, qkx_spinor_s *out, const qkx_spinor_s *e, const qkx_gauge_s *U, double *lpart)
+{
+    const Geom g = qkx::make_geom(U->L, U->bc);
+    const GaugeF18 G = make_gauge<GaugeF18>(U);
+    int nb = layer_blocks(g.V);
+    const int nblk8 = net_remap(nb);
+    const Hid hid = hid_of(n->fh, g.V);
+    return with_ch(n, [&](auto CHC) {
+        constexpr int CH = decltype(CHC)::value;
+        return with_bf(n, [&](auto BFC) {
+            constexpr bool BF = decltype(BFC)::value;
+            const LayerWeights<CH, 4, false, BF> w{BF ? (const void *)(n->wb + n->n1) : (const void *)(n->w + n->n1)};
+            if (e)
+                return with_spinor(e, [&](auto E) {
+                    hipLaunchKernelGGL((net_contract_kernel<CH, BF, true, SpinorF, decltype(E)>), dim3(nb),
+                                       dim3(kLayerT), 0, qkx::g_stream, hid, SpinorF{n->gout, g.V}, E, G, g, nblk8,
+                                       w, lpart);
+                    QKX_HIP(hipGetLastError());
+                    return QKX_SUCCESS;
+                });
+            return with_spinor(out, [&](auto S) {
+                hipLaunchKernelGGL((net_contract_kernel<CH, BF, false, decltype(S), decltype(S)>), dim3(nb),
+                                   dim3(kLayerT), 0, qkx::g_stream, hid, S, S, G, g, nblk8, w, (double *)nullptr);
+                QKX_HIP(hipGetLastError());
+                return QKX_SUCCESS;
+            });
+        });
+    });
+}
+
+// Z of a hidden field and a spinor (v) or the loss gradient (v null)
+int launch_wgrad(qkx_net_s *n, Hid f, const qkx_spinor_s *v, const qkx_gauge_s *U, double *part, int bs, int nb)
+{
+    const Geom g = qkx::make_geom(U->L, U->bc);
+    const GaugeF18 G = make_gauge<GaugeF18>(U);
+    return with_ch(n, [&](auto CHC) {
+        constexpr int CH = decltype(CHC)::value;
+        auto go = [&](auto S) {
+            hipLaunchKernelGGL((net_wgrad_kernel<CH, decltype(S)>), dim3(nb, wgrad_groups(CH)), dim3(bs), 0,
+                               qkx::g_stream, f, S, G, g, part);
+            QKX_HIP(hipGetLastError());
+            return QKX_SUCCESS;
+        };
+        if (v) return with_spinor(v, go);
+        return go(SpinorF{n->gout, g.V});
+    });
 }
 
 } // namespace
@@ -753,53 +595,8 @@ int net_apply(qkx_net_s *n, qkx_spinor_s *out, const qkx_spinor_s *in, const qkx
     int rc;
     if ((rc = check_net_gauge(U)) || (rc = check_spinor(in, U)) || (rc = check_spinor(out, U))) return rc;
     if ((rc = net_buffers(n, U->L))) return rc;
-    if ((rc = to_feat(in, n->fin))) return rc;
-    if ((rc = net_forward(n, U))) return rc;
-    return from_feat(n->fout, out);
-}
-// The even-odd weight tables from the current weights (BF16 copies when
-// the network runs in BF16); a solve prepares them once.
-int net_prep_eo(qkx_net_s *n)
-{
-    const int T = eo_table(n->ch);
-    if (!n->weo) QKX_HIP(hipMalloc(&n->weo, sizeof(float2) * 2 * T));
-    hipLaunchKernelGGL(eo_weights_kernel, dim3((2 * T + 255) / 256), dim3(256), 0, qkx::g_stream, n->w, n->wb,
-                       n->bf16, n->ch, n->weo);
-    QKX_HIP(hipGetLastError());
-    return QKX_SUCCESS;
-}
-
-// out = N_e in (adjoint: N_e^dag in) on even-parity fields of one precision
-// and batch size; net_prep_eo must have run since the weights last changed.
-// out may be in.  skip (optional, device): both launches return at once
-// while *skip != 0.
-int net_apply_eo(qkx_net_s *n, qkx_spinor_s *out, const qkx_spinor_s *in, const qkx_gauge_s *U, int adjoint,
-                 const int *skip)
-{
-    int rc;
-    if ((rc = check_net_gauge(U))) return rc;
-    if (in->subset != QKX_SUBSET_EVEN || out->subset != QKX_SUBSET_EVEN || in->prec != out->prec ||
-        in->nrhs != out->nrhs || in->L[0] != U->L[0] || in->L[1] != U->L[1] || in->L[2] != U->L[2] ||
-        in->L[3] != U->L[3] || out->L[0] != U->L[0] || out->L[1] != U->L[1] || out->L[2] != U->L[2] ||
-        out->L[3] != U->L[3]) {
-        qkx::set_error("net (even-odd): in and out must be even-parity fields of one precision and batch size on "
-                       "the gauge's lattice");
-        return QKX_ERR_ARG;
-    }
-    const size_t need = (size_t)n->ch * 3 * (size_t)in->Vh * eo_chunk(n, in);
-    if (need > n->ehid_cap) {
-        if (n->ehid) (void)hipFree(n->ehid);
-        n->ehid = nullptr;
-        n->ehid_cap = 0;
-        QKX_HIP(hipMalloc(&n->ehid, sizeof(float2) * need));
-        n->ehid_cap = need;
-    }
-    return dispatch_prec(in->prec, [&](auto tag) {
-        using S = decltype(tag);
-        if (n->ch == 16) return launch_eo<16, S>(n, out, in, U, adjoint, skip);
-        if (n->ch == 4) return launch_eo<4, S>(n, out, in, U, adjoint, skip);
-        return launch_eo<8, S>(n, out, in, U, adjoint, skip);
-    });
+    if ((rc = launch_expand<false>(n, in, nullptr, hid_of(n->fh, U->V), U))) return rc;
+    return launch_contract(n, out, nullptr, U, nullptr);
 }
 } // namespace qkx
 
@@ -840,8 +637,8 @@ int qkx_net_create(qkx_net **out, int ch)
 int qkx_net_destroy(qkx_net *n)
 {
     if (!n) return QKX_SUCCESS;
-    void *ptrs[] = {n->w,    n->wb, n->grad, n->m,  n->v,    n->loss, n->fin,
-                    n->fh,   n->fout, n->gout, n->gh, n->part, n->weo, n->ehid};
+    void *ptrs[] = {n->w,  n->wb,   n->grad, n->m,    n->v,   n->loss,
+                    n->fh, n->gout, n->gh,   n->part, n->weo, n->ehid};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     delete n;
@@ -852,7 +649,7 @@ int qkx_net_release_buffers(qkx_net *n)
 {
     QKX_CHECK_ARG(n, "qkx_net_release_buffers: null argument");
     QKX_HIP(hipStreamSynchronize(qkx::g_stream));   // no launch may still use them
-    float2 **bufs[6] = {&n->fin, &n->fh, &n->fout, &n->gout, &n->gh, &n->ehid};
+    float4 **bufs[4] = {&n->fh, &n->gout, &n->gh, &n->ehid};
     for (auto b : bufs) {
         if (*b) (void)hipFree(*b);
         *b = nullptr;
@@ -928,30 +725,21 @@ int qkx_net_accumulate_grad(qkx_net *n, const qkx_spinor *r, const qkx_spinor *e
     if ((rc = check_net_gauge(U)) || (rc = check_spinor(r, U)) || (rc = check_spinor(e, U))) return rc;
     if ((rc = net_buffers(n, U->L))) return rc;
     const int V = U->V;
-    if ((rc = to_feat(r, n->fin))) return rc;
-    if ((rc = net_forward(n, U))) return rc;
-    // target into gh's first 4 channels (free until the adjoint below)
-    if ((rc = to_feat(e, n->gh))) return rc;
-    const int ne = 12 * V, nb = std::min(nblk(ne), 1024);
-    hipLaunchKernelGGL(loss_kernel, dim3(nb), dim3(kT), 0, qkx::g_stream, n->fout, n->gh, n->gout, ne, n->part);
-    hipLaunchKernelGGL(loss_finish_kernel, dim3(1), dim3(64), 0, qkx::g_stream, n->part, nb, n->loss);
+    int bs, nb;
+    grad_grid(n->ch, V, bs, nb);
+    const size_t nz = (size_t)nb * 9 * 4 * n->ch * 2;
+    double *z1 = n->part, *z2 = z1 + nz, *lpart = z2 + nz;
+    const Hid fh = hid_of(n->fh, V), gh = hid_of(n->gh, V);
+    const SpinorF gout{n->gout, V};
+    if ((rc = launch_expand<false>(n, r, nullptr, fh, U))) return rc;
+    if ((rc = launch_contract(n, nullptr, e, U, lpart))) return rc;
+    if ((rc = launch_wgrad(n, fh, nullptr, U, z2, bs, nb))) return rc;
+    if ((rc = launch_expand<true>(n, nullptr, &gout, gh, U))) return rc;
+    if ((rc = launch_wgrad(n, gh, r, U, z1, bs, nb))) return rc;
+    hipLaunchKernelGGL(grad_finish_kernel, dim3(2 * 9 * 4 * n->ch + 1), dim3(64), 0, qkx::g_stream, z1, z2, nb, lpart,
+                       loss_blocks(V), n->ch, n->grad, n->loss);
     QKX_HIP(hipGetLastError());
-    const bool bf = n->bf16 != 0;
-    const void *w2 = bf ? (const void *)(n->wb + n->n1) : (const void *)(n->w + n->n1);
-    double2 *g1 = n->grad, *g2 = n->grad + n->n1;
-    if (n->ch == 16) {
-        if ((rc = launch_wgrad<16, 4>(n->gout, n->fh, U, n, g2))) return rc;
-        if ((rc = launch_ptc<4, 16, true>(n->gout, n->gh, U, w2, bf))) return rc;
-        return launch_wgrad<4, 16>(n->gh, n->fin, U, n, g1);
-    }
-    if (n->ch == 4) {
-        if ((rc = launch_wgrad<4, 4>(n->gout, n->fh, U, n, g2))) return rc;
-        if ((rc = launch_ptc<4, 4, true>(n->gout, n->gh, U, w2, bf))) return rc;
-        return launch_wgrad<4, 4>(n->gh, n->fin, U, n, g1);
-    }
-    if ((rc = launch_wgrad<8, 4>(n->gout, n->fh, U, n, g2))) return rc;
-    if ((rc = launch_ptc<4, 8, true>(n->gout, n->gh, U, w2, bf))) return rc;
-    return launch_wgrad<4, 8>(n->gh, n->fin, U, n, g1);
+    return QKX_SUCCESS;
 }
 
 int qkx_net_read_grad(qkx_net *n, float *g, double *loss)
