@@ -534,7 +534,7 @@ template <class SX, class SR, class SP, bool UPDX = true> struct CgFin {
     // every lane), then the waves in order
     template <class A> __device__ __forceinline__ void begin(const A &)
     {
-        __shared__ double lh[4], ll[4];
+        __shared__ double lh[8], ll[8];   // up to 512 threads
         DD v{0.0, 0.0};
         for (int i = threadIdx.x; i < npap; i += blockDim.x) v = dd_add(v, pap_part[i]);
         v = dd_wave_sum(v);
@@ -773,6 +773,201 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HopWaves<SI
     Epi ep = a.epi[0];                 // uniform (scalar) load for a single rhs
     if (a.nrhs > 1) ep = a.epi[u - fdiv(u, a.dnr) * a.nrhs];
     hop_body<B, DAG, AUX, DEPTH>(a, fin, blockIdx.x, p, u, ep);
+}
+
+// xi = U h of one direction (the boundary sign on h), the products and sums of
+// apply_dir.
+template <int B, int MU, int KIND, bool DAGL, class SIn, class G, class T>
+__device__ __forceinline__ void dir_xi(Cx<T> xi[6], const SIn &in, const G &U, const HopOps<SIn, G> &o, T sign)
+{
+    Cx<T> psi[12];
+    in.template unpack<spin_mask<B, MU, KIND>()>(o.psi, psi);
+    Cx<T> h[6];
+    project_k<B, MU, KIND, 0>(psi, h);
+    project_k<B, MU, KIND, 1>(psi, h);
+    Cx<T> Ul[9];
+    U.unpack(o.link, Ul);
+    if (sign != T(1)) {
+#pragma unroll
+        for (int k = 0; k < 6; k++) h[k] = sign * h[k];
+    }
+    link_mul<DAGL, false>(Ul, h, xi);
+}
+
+// FP64 hop of a small lattice, one right-hand side: eight wavefronts per 64
+// sites, wavefront w the direction w (+x -x +y -y +z -z +t -t), so that the
+// gathers of a site are all in flight at once and eight times as many
+// wavefronts are resident.  The half spinors meet in LDS (48 KB); wavefront w
+// < 6 then sums spins (w / 3, w / 3 + 2) -- the two that gamma5 pairs -- of
+// colour w % 3 over the directions, in hop_body's order, and finishes them.
+// With one thread per site a lattice of 8^3x16 is 128 wavefronts on 1024
+// SIMDs, each a chain of eight gathers: tm 9.4 -> 4.7 us, even-odd normal
+// operator (4 hops) 33.9 -> 19.1 us, with the same bits.
+constexpr int kSplitT = 512;
+template <int B, int FW, int S, class T>
+__device__ __forceinline__ Cx<T> split_sum(const double2 (*xi)[6][64], int c, int lane)
+{
+    Cx<T> R{T(0), T(0)};
+    auto add = [&](auto MUC, auto KINDC, int d) {
+        constexpr Proj P = kProj[B][decltype(MUC)::value][decltype(KINDC)::value];
+        if constexpr (P.q[S] != K0) {
+            const double2 v = xi[d][P.kq[S] * 3 + c][lane];
+            R = R + umul<P.q[S]>(Cx<T>{v.x, v.y});
+        }
+    };
+    using F = std::integral_constant<int, FW>;
+    using Bk = std::integral_constant<int, 1 - FW>;
+    add(std::integral_constant<int, 0>{}, F{}, 0);
+    add(std::integral_constant<int, 0>{}, Bk{}, 1);
+    add(std::integral_constant<int, 1>{}, F{}, 2);
+    add(std::integral_constant<int, 1>{}, Bk{}, 3);
+    add(std::integral_constant<int, 2>{}, F{}, 4);
+    add(std::integral_constant<int, 2>{}, Bk{}, 5);
+    add(std::integral_constant<int, 3>{}, F{}, 6);
+    add(std::integral_constant<int, 3>{}, Bk{}, 7);
+    return R;
+}
+
+template <class G, int B, bool DAG, bool AUX, class Fin = StoreFin>
+__global__ __launch_bounds__(kSplitT) void hop_split_kernel(HopArgs<SpinorD, SpinorD, SpinorD, G> a, Fin fin)
+{
+    using T = double;
+    constexpr bool CG = !std::is_same_v<Fin, StoreFin>;
+    if (a.skip && *a.skip) return;   // uniform over the grid
+    __shared__ double2 xi_s[8][6][64];
+    __shared__ double nrm_s[8];
+    const Geom &g = a.g;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+    // blocks per parity are whole multiples of 8 when nblk8 > 0 (hop_unit's order)
+    int p, lb;
+    if (a.par_out >= 0) {
+        p = a.par_out;
+        lb = logical_block(blockIdx.x, a.nblk8);
+    } else if (a.nblk8 > 0) {
+        const int i = blockIdx.x >> 3;
+        p = i & 1;
+        lb = (blockIdx.x & 7) * a.nblk8 + (i >> 1);
+    } else {
+        p = blockIdx.x & 1;
+        lb = blockIdx.x >> 1;
+    }
+    const int v = lb * 64 + lane;
+    const bool live = v < g.Vh;
+    const int cb = min(v, g.Vh - 1);
+    const HopSite hs = hop_site(g, p, cb);
+    const int qoff = (p ^ 1) * g.Vh, poff = p * g.Vh;
+    const int in_q = a.in_off[p ^ 1];
+    constexpr int FW = DAG ? 1 : 0, BW = DAG ? 0 : 1;
+    // the epilogue's operands of wavefront w < 6, requested with the gathers
+    const int c = w % 3, k0 = (w / 3) * 3 + c, k1 = k0 + 6;
+    Cx<T> x0{0, 0}, x1{0, 0};
+    if (AUX && w < 6) {
+        const double2 *q = a.aux.p + a.aux_off[p] + cb;
+        const double2 u0 = q[(size_t)k0 * a.aux.stride], u1 = q[(size_t)k1 * a.aux.stride];
+        x0 = {u0.x, u0.y};
+        x1 = {u1.x, u1.y};
+    }
+    Cx<T> xi[6];
+    auto dir = [&](auto MUC, auto KINDC, auto BACK, int nb, T sign) {
+        constexpr int MU = decltype(MUC)::value, KIND = decltype(KINDC)::value;
+        constexpr bool BK = decltype(BACK)::value;
+        const auto o = fetch_dir<B, MU, KIND>(a.in, in_q + nb, a.U, BK ? qoff + nb : poff + cb);
+        dir_xi<B, MU, KIND, BK>(xi, a.in, a.U, o, sign);
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+    using IF = std::integral_constant<int, FW>;
+    using IB = std::integral_constant<int, BW>;
+    const T bc = T(g.bc);
+    switch (w) {
+    case 0: dir(I0{}, IF{}, std::false_type{}, hs.nb[0], T(1)); break;
+    case 1: dir(I0{}, IB{}, std::true_type{}, hs.nb[1], T(1)); break;
+    case 2: dir(I1{}, IF{}, std::false_type{}, hs.nb[2], T(1)); break;
+    case 3: dir(I1{}, IB{}, std::true_type{}, hs.nb[3], T(1)); break;
+    case 4: dir(I2{}, IF{}, std::false_type{}, hs.nb[4], T(1)); break;
+    case 5: dir(I2{}, IB{}, std::true_type{}, hs.nb[5], T(1)); break;
+    case 6: dir(I3{}, IF{}, std::false_type{}, hs.nb[6], hs.tw_p ? bc : T(1)); break;
+    default: dir(I3{}, IB{}, std::true_type{}, hs.nb[7], hs.tw_m ? bc : T(1)); break;
+    }
+#pragma unroll
+    for (int k = 0; k < 6; k++) xi_s[w][k][lane] = make_double2(xi[k].re, xi[k].im);
+    if constexpr (CG) fin.begin(a);   // ends in a barrier
+    __syncthreads();
+    double nrm2 = 0.0;
+    if (w < 6 && live) {
+        // spins j and j + 2 of colour c: gamma5 exchanges them (UKQCD), or
+        // keeps the first and negates the second (chiral)
+        Cx<T> R0, R1;
+        if (w < 3) {
+            R0 = split_sum<B, FW, 0, T>(xi_s, c, lane);
+            R1 = split_sum<B, FW, 2, T>(xi_s, c, lane);
+        } else {
+            R0 = split_sum<B, FW, 1, T>(xi_s, c, lane);
+            R1 = split_sum<B, FW, 3, T>(xi_s, c, lane);
+        }
+        const Epi &e = a.epi[0];
+        auto g5 = [](Cx<T> u0, Cx<T> u1, Cx<T> &v0, Cx<T> &v1) {
+            if constexpr (B == QKX_BASIS_UKQCD) {
+                v0 = u1;
+                v1 = u0;
+            } else {
+                v0 = u0;
+                v1 = {-u1.re, -u1.im};
+            }
+        };
+        Cx<T> h0, h1, y0, y1, o0, o1;
+        g5(R0, R1, h0, h1);
+        g5(x0, x1, y0, y1);
+        auto fin1 = [&](Cx<T> R, Cx<T> h, Cx<T> x, Cx<T> y) {
+            T re = fma(e.gR, -h.im, e.cR * R.re), im = fma(e.gR, h.re, e.cR * R.im);
+            if (AUX) {
+                re = fma(e.gX, -y.im, fma(e.cX, x.re, re));
+                im = fma(e.gX, y.re, fma(e.cX, x.im, im));
+            }
+            return Cx<T>{re, im};
+        };
+        o0 = fin1(R0, h0, x0, y0);
+        o1 = fin1(R1, h1, x1, y1);
+        if (e.g5out) {
+            g5(o0, o1, h0, h1);
+            o0 = h0;
+            o1 = h1;
+        }
+        const int so = a.out_off[p] + cb;
+        if constexpr (CG) {
+            auto upd = [&](int k, Cx<T> o) {
+                double2 *xp = fin.x.p + (size_t)k * fin.x.stride + so, *rp = fin.r.p + (size_t)k * fin.r.stride + so;
+                double2 xv = *xp, rv = *rp;
+                const double2 pv = fin.p.p[(size_t)k * fin.p.stride + so];
+                xv = make_double2(xv.x + fin.alpha * pv.x, xv.y + fin.alpha * pv.y);
+                rv = make_double2(rv.x - fin.alpha * o.re, rv.y - fin.alpha * o.im);
+                *xp = xv;
+                *rp = rv;
+                nrm2 += rv.x * rv.x + rv.y * rv.y;
+            };
+            upd(k0, o0);
+            upd(k1, o1);
+        } else {
+            a.out.p[(size_t)k0 * a.out.stride + so] = make_double2(o0.re, o0.im);
+            a.out.p[(size_t)k1 * a.out.stride + so] = make_double2(o1.re, o1.im);
+            nrm2 = o0.re * o0.re + o0.im * o0.im + o1.re * o1.re + o1.im * o1.im;
+        }
+    }
+    double *dst = nullptr;
+    if constexpr (CG) dst = fin.r2_part;
+    else dst = a.norm_partial;
+    if (!dst) return;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) nrm2 += __shfl_xor(nrm2, off, 64);
+    if (lane == 0) nrm_s[w] = nrm2;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0;
+        for (int i = 0; i < 6; i++) t += nrm_s[i];
+        dst[blockIdx.x] = t;
+    }
 }
 
 // Single-RHS FP16 half-lattice hop with the x and y neighbours staged in
@@ -1429,6 +1624,12 @@ bool share_links_for(int nrhs, long units)
 // 0: checkerboard index order; 1: blocked walk (HopTrav) for every hop;
 // 2: blocked walk for the full-lattice FP64 hops only
 int g_site_order = QKX_SITE_ORDER_DEFAULT;
+// FP64 single-RHS hops of at most this many output sites split each site's
+// directions over eight wavefronts (hop_split_kernel).  tm 13.3 -> 11.6 us at
+// 12^3x32 and 31.4 -> 27.6 us at 16^3x32 (131,072 sites); even-odd normal operator
+// 81.3 -> 74.9 us there (65,536 sites a hop) and equal (57.3 us) at 16^3x24.  Beyond,
+// one thread per site fills the SIMDs and has the half spinors in registers.
+constexpr int kSplitSites = 131072;
 #ifndef QKX_STAGE_DEFAULT
 #define QKX_STAGE_DEFAULT 0
 #endif
@@ -1611,6 +1812,33 @@ int launch_hop_t(qkx_spinor_s *out, const qkx_spinor_s *in, const qkx_spinor_s *
                 sh = it->second.shape;
                 if (g_share_links != 1) sh.share = dshare;   // an explicit setting wins
             }
+        }
+    }
+    // small FP64 lattices, unless the autotuner timed this kind or a candidate is being timed
+    constexpr bool split64 = std::is_same_v<S, SpinorD> &&
+                             (store || std::is_same_v<Fin, CgFin<SpinorD, SpinorD, SpinorD, true>>);
+    if constexpr (split64) {
+        if (a.nrhs == 1 && sites_out <= kSplitSites && !g_force && g_autotune != 2) {
+            int nbh = (a.g.Vh + 63) / 64;   // blocks per parity
+            a.nblk8 = 0;
+            if (g_xcd_remap && nbh >= 64) {
+                nbh = (nbh + 7) / 8 * 8;
+                a.nblk8 = nbh / 8;
+            }
+            const dim3 grid(par_out < 0 ? 2 * nbh : nbh), blk(kSplitT);
+            if (nblocks_out) *nblocks_out = grid.x;
+            double by = (double)sites_out * ((par_out < 0 ? 4 : 8) * 16.0 * (U->recon == QKX_RECON_18 ? 9 : 6) + 384.0);
+            if (aux && aux != in) by += (double)sites_out * 192.0;
+            if constexpr (!store) by += (double)sites_out * 5 * 192.0;
+            qkx::prof_begin();
+#define QKX_LAUNCH_SPLIT(DG, AX) \
+    hipLaunchKernelGGL((hop_split_kernel<G, B, DG, AX, Fin>), grid, blk, 0, qkx::g_stream, a, fin)
+            if (dagger) { if (aux) QKX_LAUNCH_SPLIT(true, true); else if constexpr (store) QKX_LAUNCH_SPLIT(true, false); }
+            else        { if (aux) QKX_LAUNCH_SPLIT(false, true); else if constexpr (store) QKX_LAUNCH_SPLIT(false, false); }
+#undef QKX_LAUNCH_SPLIT
+            qkx::prof_end(by, in->prec);
+            QKX_HIP(hipGetLastError());
+            return QKX_SUCCESS;
         }
     }
     const bool few = a.nrhs < 8;   // 3-7 RHS: the larger site capacity

@@ -97,6 +97,37 @@ __device__ double block_sum_array(const double *v, int n)
     return dd_value(r);
 }
 
+// block_sum_array of two arrays at once (the same bits): the two chains of
+// dependent additions overlap, and the barriers are shared.
+__device__ void block_sum_arrays(const double *v, int n, const double *u, int m, double &sv, double &su)
+{
+    __shared__ double l[4][kThreads / 64];
+    DD s{0.0, 0.0}, t{0.0, 0.0};
+    for (int i = threadIdx.x; i < n; i += blockDim.x) s = dd_add(s, v[i]);
+    for (int i = threadIdx.x; i < m; i += blockDim.x) t = dd_add(t, u[i]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        s = dd_add(s, DD{__shfl_xor(s.hi, off, 64), __shfl_xor(s.lo, off, 64)});
+        t = dd_add(t, DD{__shfl_xor(t.hi, off, 64), __shfl_xor(t.lo, off, 64)});
+    }
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+        l[0][w] = s.hi;
+        l[1][w] = s.lo;
+        l[2][w] = t.hi;
+        l[3][w] = t.lo;
+    }
+    __syncthreads();
+    DD r{l[0][0], l[1][0]}, q{l[2][0], l[3][0]};
+    for (int i = 1; i < (int)(blockDim.x >> 6); i++) {
+        r = dd_add(r, DD{l[0][i], l[1][i]});
+        q = dd_add(q, DD{l[2][i], l[3][i]});
+    }
+    __syncthreads();   // l is reused by the next call
+    sv = dd_value(r);
+    su = dd_value(q);
+}
+
 // out[0] = sum(part[0..n)), compensated, in a fixed order, by one workgroup
 __global__ __launch_bounds__(1024) void sum_partials_kernel(const double *part, int n, double *out)
 {
@@ -208,11 +239,12 @@ __global__ __launch_bounds__(kThreads) void cg_dir_kernel(S p, SR r, SX x, int n
         r.load(s, rv);
         if (HASX && mode == 0) x.load(s, xv);
     }
-    const double r2n = block_sum_array(r2_part, nr2);
+    double r2n, pap = 0;
+    if (mode == 0) block_sum_arrays(r2_part, nr2, pap_part, npap, r2n, pap);
+    else r2n = block_sum_array(r2_part, nr2);
     double beta;
     int flag = 0;
     if (mode == 0) {
-        const double pap = block_sum_array(pap_part, npap);
         if constexpr (HASX) {
             if (s < n) {
                 const TX ax = TX(cur->r2 / pap);
@@ -242,6 +274,41 @@ __global__ __launch_bounds__(kThreads) void cg_dir_kernel(S p, SR r, SX x, int n
         out[k] = {(typename S::Real)(rv[k].re + b * T(pv[k].re)), (typename S::Real)(rv[k].im + b * T(pv[k].im))};
     p.store(s, out);
 }
+
+// Mode 0 of cg_dir_kernel for FP64 p and r of a small lattice, one thread per
+// complex number (the 12 component arrays of n sites are one array of 12 n):
+// with one thread per site, 8192 sites are 32 workgroups, each thread a chain
+// of 24 loads.  With hop_split_kernel, FP64 CG at 8^3x16 (528 iterations):
+// 15.6 -> 10.4 ms.
+__global__ __launch_bounds__(kThreads) void cg_dir_small_kernel(double2 *p, const double2 *r, int n12, const CGSlot *cur,
+                                                                CGSlot *next, const double *r2_part, int nr2,
+                                                                const double *pap_part, int npap, double stop2,
+                                                                double delta2)
+{
+    if (cur->flag) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *next = *cur;
+        return;
+    }
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    double2 pv = make_double2(0, 0), rv = pv;
+    if (i < n12) {
+        pv = p[i];
+        rv = r[i];
+    }
+    double r2n, pap;
+    block_sum_arrays(r2_part, nr2, pap_part, npap, r2n, pap);
+    int flag = 0;
+    if (!(pap > 0.0) || !isfinite(r2n)) flag = 3;
+    else if (r2n <= stop2) flag = 2;
+    else if (r2n < delta2 * cur->maxr2) flag = 1;
+    const double beta = r2n / cur->r2;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *next = CGSlot{r2n, cur->r2, pap, cur->maxr2, flag, cur->k + 1};
+    if (flag || i >= n12) return;
+    p[i] = make_double2(rv.x + beta * pv.x, rv.y + beta * pv.y);
+}
+// At most this many sites: 768 workgroups, each summing 2 x 256 partials; with
+// more, one thread per site fills the CUs and repeats the sums less often.
+constexpr int kDirSmallSites = 16384;
 
 // every workgroup sums v[0..n) with block_sum_array and writes its result
 __global__ __launch_bounds__(kThreads) void block_sum_probe_kernel(const double *v, int n, double *out)
@@ -397,6 +464,12 @@ int enqueue_dir(Engine &E, qkx_spinor_s *r, qkx_spinor_s *p, const qkx::CgFuse &
             QKX_HIP(hipGetLastError());
             return QKX_SUCCESS;
         }
+    } else if (n <= kDirSmallSites) {
+        hipLaunchKernelGGL(cg_dir_small_kernel, dim3(nblk(12 * n)), dim3(kThreads), 0, qkx::g_stream, P.p,
+                           make_spinor<SR>(r).p, 12 * n, E.cur(), E.next(), r2_src, nr2, f.pap_part, f.npap, E.stop2,
+                           E.delta2);
+        QKX_HIP(hipGetLastError());
+        return QKX_SUCCESS;
     }
     hipLaunchKernelGGL((cg_dir_kernel<S, SR, S, false>), dim3(nblk(n)), dim3(kThreads), 0, qkx::g_stream, P,
                        make_spinor<SR>(r), P, n, E.cur(), E.next(), r2_src, nr2, f.pap_part, f.npap, E.stop2, E.delta2,
@@ -949,7 +1022,7 @@ static int cg_impl(qkx_spinor *x, const qkx_spinor *b, const qkx_gauge *U, const
     QKX_CHECK_ARG(x->prec == QKX_PREC_DOUBLE && b->prec == QKX_PREC_DOUBLE && U->prec == QKX_PREC_DOUBLE,
                   "qkx_cg: FP64 fields required");
     QKX_CHECK_ARG(x->subset == QKX_SUBSET_FULL && b->subset == QKX_SUBSET_FULL, "qkx_cg: full fields required");
-    if (int rc = ensure_state(b->V / kThreads + 64)) return rc;
+    if (int rc = ensure_state(b->V / 64 + 64)) return rc;
     auto t0 = std::chrono::steady_clock::now();
     NormalOp A{U, p->kappa, 2.0 * p->kappa * p->mu * p->twistSign, 1.0 + 4.0 * p->kappa * p->kappa * p->mu * p->mu,
                false, nullptr, nullptr, nullptr};
@@ -1082,7 +1155,7 @@ int qkx_solve(qkx_spinor *x, const qkx_spinor *b, const qkx_gauge *U, const qkx_
                   "qkx_solve: x and b must be full FP64 fields");
     QKX_CHECK_ARG(U->prec == QKX_PREC_DOUBLE && U->recon == QKX_RECON_18, "qkx_solve: U must be FP64 recon 18");
     QKX_CHECK_ARG(o->tol > 0 && o->maxIter > 0, "qkx_solve: bad tol/maxIter");
-    if (int rc = ensure_state(b->V / kThreads + 64)) return rc;
+    if (int rc = ensure_state(b->V / 64 + 64)) return rc;
     auto t0 = std::chrono::steady_clock::now();
     const int *L = b->L;
     const bool mixed = o->inner_prec != QKX_PREC_DOUBLE;
