@@ -257,8 +257,6 @@ struct Hid {
         }
     }
 };
-    }
-};
 
 // One layer 4 -> CH for one unit: adds the paths P .. P1 - 1 of the mixed
 // transports of the four input vectors.  unit(s) is the input field's entry of
