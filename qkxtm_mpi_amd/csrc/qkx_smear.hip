@@ -93,93 +93,49 @@ struct ProjConst {
     double r18, r12, r23, s3;
 };
 
-// sin and cos for |x| <= pi/3 by their Taylor series (the first dropped terms
-// are below 1e-19): the projection's angles are thirds of arguments, so the
-// library's reduction of large arguments is not needed.
-__device__ __forceinline__ void sincos_third(double x, double &sn, double &cs)
-{
-    const double y = x * x;
-    double s = 1.0 / 121645100408832000.0, c = 1.0 / 2432902008176640000.0;   // 1/19!, 1/20!
-    s = fma(-s, y, 1.0 / 355687428096000.0);                                  // 1/17!
-    c = fma(-c, y, 1.0 / 6402373705728000.0);                                 // 1/18!
-    s = fma(-s, y, 1.0 / 1307674368000.0);
-    c = fma(-c, y, 1.0 / 20922789888000.0);
-    s = fma(-s, y, 1.0 / 6227020800.0);
-    c = fma(-c, y, 1.0 / 87178291200.0);
-    s = fma(-s, y, 1.0 / 39916800.0);
-    c = fma(-c, y, 1.0 / 479001600.0);
-    s = fma(-s, y, 1.0 / 362880.0);
-    c = fma(-c, y, 1.0 / 3628800.0);
-    s = fma(-s, y, 1.0 / 5040.0);
-    c = fma(-c, y, 1.0 / 40320.0);
-    s = fma(-s, y, 1.0 / 120.0);
-    c = fma(-c, y, 1.0 / 720.0);
-    s = fma(-s, y, 1.0 / 6.0);
-    c = fma(-c, y, 1.0 / 24.0);
-    c = fma(-c, y, 0.5);
-    sn = fma(-s * y, x, x);
-    cs = fma(-c, y, 1.0);
-}
-// a0 b0 + a1 b1 + a2 b2, the same with conjugated a's, and a x b conjugated
-__device__ __forceinline__ C dot3(C a0, C b0, C a1, C b1, C a2, C b2)
-{
-    return cmac(cmac(cmul_f(a0, b0), a1, b1), a2, b2);
-}
-__device__ __forceinline__ C cdot3(C a0, C b0, C a1, C b1, C a2, C b2)
-{
-    return cjmac(cjmac(cjmul_f(a0, b0), a1, b1), a2, b2);
-}
-__device__ __forceinline__ C ccross(C a, C d, C b, C c)   // conj(a d - b c)
-{
-    const C nb = {-b.re, -b.im};
-    return conjc(cmac(cmul_f(a, d), nb, c));
-}
-__device__ __forceinline__ C axpyc(C x, C a, C v)   // x - a v
-{
-    const C na = {-a.re, -a.im};
-    return cmac(x, na, v);
-}
-__device__ __forceinline__ double nrm3(C a, C b, C c)
-{
-    return fma(a.re, a.re, fma(a.im, a.im, fma(b.re, b.re, fma(b.im, b.im, fma(c.re, c.re, c.im * c.im)))));
-}
-
 // SU(3) projection of one matrix: U = M (M^dag M)^{-1/2} exp(-i arg(det M)/3)
 // by the reference's closed-form eigensystem of H = M^dag M (Cardano roots of
 // the traceless part, eigenvectors from two rows of H - e), then Gram-Schmidt
 // of columns 1-2 and column 3 = conj(col1 x col2).  If the off-diagonal moduli
 // of H sum to at most 1e-8, row i of M is scaled by 1/sqrt(H_ii) instead.
-//
-// The steps follow lib/blas.cpp:32-420, the eigenvalues operation by operation:
-// they are ill-conditioned where H is nearly degenerate (the trigonometric form
-// of the real roots, exact to 1e-15 there, leaves the reference by 2e-12 on
-// generic matrices), so results agree to rounding only if they are formed alike.
+// The steps follow lib/blas.cpp:32-420 so that results agree to rounding.
 __device__ void su3_project(Mat &M, const ProjConst &pc)
 {
-    C *m = M.a;
-    const C c0 = axpyc(cmul_f(m[4], m[8]), m[5], m[7]), c1 = axpyc(cmul_f(m[5], m[6]), m[3], m[8]),
-            c2 = axpyc(cmul_f(m[3], m[7]), m[4], m[6]);
-    const C det = dot3(m[0], c0, m[1], c1, m[2], c2);
+    const C *m = M.a;
+    C det = cmul(m[0], cmul(m[4], m[8])) + cmul(m[1], cmul(m[5], m[6])) + cmul(m[2], cmul(m[3], m[7]));
+    det = det - (cmul(m[2], cmul(m[4], m[6])) + cmul(m[0], cmul(m[5], m[7])) + cmul(m[1], cmul(m[3], m[8])));
     const double phase = atan2(det.im, det.re) / 3.0;
 
-    const double H00 = nrm3(m[0], m[3], m[6]), H11 = nrm3(m[1], m[4], m[7]), H22 = nrm3(m[2], m[5], m[8]);
-    const C h01 = cdot3(m[0], m[1], m[3], m[4], m[6], m[7]), h02 = cdot3(m[0], m[2], m[3], m[5], m[6], m[8]),
-            h12 = cdot3(m[1], m[2], m[4], m[5], m[7], m[8]);
-    const double n01 = nrm2c(h01), n02 = nrm2c(h02), n12 = nrm2c(h12);
+    C H[9];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) H[3 * i + j] = cjmul(m[i], m[j]) + cjmul(m[3 + i], m[3 + j]) + cjmul(m[6 + i], m[6 + j]);
+    // exact Hermiticity of the off-diagonal pairs
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = i + 1; j < 3; j++) {
+            C h = {(H[3 * i + j].re + H[3 * j + i].re) * 0.5, (H[3 * i + j].im - H[3 * j + i].im) * 0.5};
+            H[3 * i + j] = h;
+            H[3 * j + i] = conjc(h);
+        }
+    const double n01 = nrm2c(H[1]), n02 = nrm2c(H[2]), n12 = nrm2c(H[5]);
     if (sqrt(n01) + sqrt(n02) + sqrt(n12) <= 1e-08) {
-        const double e[3] = {1.0 / sqrt(H00), 1.0 / sqrt(H11), 1.0 / sqrt(H22)};
 #pragma unroll
-        for (int i = 0; i < 3; i++)
+        for (int i = 0; i < 3; i++) {
+            const double e = 1.0 / sqrt(H[4 * i].re);
 #pragma unroll
-            for (int j = 0; j < 3; j++) m[3 * i + j] = e[i] * m[3 * i + j];
+            for (int j = 0; j < 3; j++) M.a[3 * i + j] = e * M.a[3 * i + j];
+        }
         return;
     }
     // eigenvalues: e^3 + a e + b = 0 for the traceless part
-    const double tr = (H00 + H11 + H22) / 3.0;
-    const double h00 = H00 - tr, h11 = H11 - tr, h22 = H22 - tr;
+    const double tr = (H[0].re + H[4].re + H[8].re) / 3.0;
+    const double h00 = H[0].re - tr, h11 = H[4].re - tr, h22 = H[8].re - tr;
     const double a = -(h22 * h22 - h00 * h11 + n01 + n02 + n12);
-    const C t1 = cmul(h01, cmul(h12, conjc(h02)));
-    const C t2 = cmul(h02, cmul(conjc(h01), conjc(h12)));
+    const C t1 = cmul(H[1], cmul(H[5], conjc(H[2])));
+    const C t2 = cmul(H[2], cmul(conjc(H[1]), conjc(H[5])));
     C b;
     b.re = (-h00 * h11 * h22 + h22 * n01 - t1.re + h11 * n02) + (h00 * n12 - t2.re);
     b.im = -t1.im - t2.im;
@@ -193,7 +149,7 @@ __device__ void su3_project(Mat &M, const ProjConst &pc)
     const C z = {-9.0 * b.re + w.re, -9.0 * b.im + w.im};
     rr = sqrt(z.re * z.re + z.im * z.im);
     th = atan2(z.im, z.re);
-    sincos_third(th / 3.0, sn, cs);
+    sincos(th / 3.0, &sn, &cs);
     const double rc = cbrt(rr);
     const C D = {rc * cs, rc * sn};
     const double dd = D.re * D.re + D.im * D.im;
@@ -209,71 +165,75 @@ __device__ void su3_project(Mat &M, const ProjConst &pc)
 
     // eigenvectors (stored conjugated, as the reference does) for e0 and e1
     C v[9];
-    const C p10_21 = {fma(h01.re, h12.re, -h01.im * h12.im), -fma(h01.re, h12.im, h01.im * h12.re)};   // conj(h01) conj(h12)
-    const C p20_01 = cjmul_f(h02, h01);
+    const double H00 = H[0].re, H11 = H[4].re;
+    const C p10_21 = cmul(H[3], H[7]), p20_01 = cmul(H[6], H[1]);
 #pragma unroll
     for (int k = 0; k < 2; k++) {
         const double ek = e[k];
-        v[3 * k + 0] = {-fma(ek - H11, h02.re, p10_21.re), fma(ek - H11, h02.im, -p10_21.im)};
-        v[3 * k + 1] = {-fma(ek - H00, h12.re, p20_01.re), fma(ek - H00, h12.im, -p20_01.im)};
-        v[3 * k + 2] = {fma(-(ek - H00), ek - H11, n01), 0.0};
+        v[3 * k + 0] = {-(ek * H[6].re - H[6].re * H11 + p10_21.re), -(ek * H[6].im - H[6].im * H11 + p10_21.im)};
+        v[3 * k + 1] = {-(p20_01.re + ek * H[7].re - H00 * H[7].re), -(p20_01.im + ek * H[7].im - H00 * H[7].im)};
+        v[3 * k + 2] = {-ek * ek + ek * H00 + n01 + ek * H11 - H00 * H11, 0.0};
     }
     // Gram-Schmidt of v1 against v0, normalise both; v2 = conj(v0 x v1)
-    double nr = nrm3(v[0], v[1], v[2]);
+    double nr = nrm2c(v[0]) + nrm2c(v[1]) + nrm2c(v[2]);
     {
-        C ov = cdot3(v[3], v[0], v[4], v[1], v[5], v[2]);
+        C ov = cmul(v[0], conjc(v[3])) + cmul(v[1], conjc(v[4])) + cmul(v[2], conjc(v[5]));
         ov = (1.0 / nr) * ov;
 #pragma unroll
-        for (int j = 0; j < 3; j++) v[3 + j] = axpyc(v[3 + j], ov, v[j]);
+        for (int j = 0; j < 3; j++) v[3 + j] = v[3 + j] - cmul(ov, v[j]);
     }
-    nr = rsqrt(nr);
+    nr = 1.0 / sqrt(nr);
 #pragma unroll
     for (int j = 0; j < 3; j++) v[j] = nr * v[j];
-    nr = rsqrt(nrm3(v[3], v[4], v[5]));
+    nr = 1.0 / sqrt(nrm2c(v[3]) + nrm2c(v[4]) + nrm2c(v[5]));
 #pragma unroll
     for (int j = 0; j < 3; j++) v[3 + j] = nr * v[3 + j];
-    v[6] = ccross(v[1], v[5], v[2], v[4]);
-    v[7] = ccross(v[2], v[3], v[0], v[5]);
-    v[8] = ccross(v[0], v[4], v[1], v[3]);
+    v[6] = conjc(cmul(v[1], v[5]) - cmul(v[2], v[4]));
+    v[7] = conjc(cmul(v[2], v[3]) - cmul(v[0], v[5]));
+    v[8] = conjc(cmul(v[0], v[4]) - cmul(v[1], v[3]));
 
-    // U = (M conj(v)^T) diag(exp(-i phase)/sqrt(e_k)) v, row by row
+    // U = (M conj(v)^T) diag(exp(-i phase)/sqrt(e_k)) v
     double ps, pcs;
-    sincos_third(phase, ps, pcs);
+    sincos(phase, &ps, &pcs);
     C vr[9];
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        const double de = rsqrt(e[k]);
+        const double de = 1.0 / sqrt(e[k]);
         const C s = {de * pcs, -de * ps};
 #pragma unroll
-        for (int j = 0; j < 3; j++) vr[3 * k + j] = cmul_f(s, v[3 * k + j]);
+        for (int j = 0; j < 3; j++) vr[3 * k + j] = cmul(s, v[3 * k + j]);
     }
+    C U[9];
 #pragma unroll
     for (int i = 0; i < 3; i++) {
         C hm[3];
 #pragma unroll
         for (int k = 0; k < 3; k++)
-            hm[k] = cdot3(v[3 * k], m[3 * i], v[3 * k + 1], m[3 * i + 1], v[3 * k + 2], m[3 * i + 2]);
+            hm[k] = cmul(m[3 * i], conjc(v[3 * k])) + cmul(m[3 * i + 1], conjc(v[3 * k + 1])) +
+                    cmul(m[3 * i + 2], conjc(v[3 * k + 2]));
 #pragma unroll
-        for (int l = 0; l < 2; l++) m[3 * i + l] = dot3(hm[0], vr[l], hm[1], vr[3 + l], hm[2], vr[6 + l]);
+        for (int l = 0; l < 3; l++) U[3 * i + l] = cmul(hm[0], vr[l]) + cmul(hm[1], vr[3 + l]) + cmul(hm[2], vr[6 + l]);
     }
     // columns: the reference subtracts (sum_i U_i0 conj U_i1)/|col0|^2 col0
     // from col1, normalises both, and sets col3 = conj(col1 x col2)
-    nr = nrm3(m[0], m[3], m[6]);
+    nr = nrm2c(U[0]) + nrm2c(U[3]) + nrm2c(U[6]);
     {
-        C ov = cdot3(m[1], m[0], m[4], m[3], m[7], m[6]);
+        C ov = cmul(U[0], conjc(U[1])) + cmul(U[3], conjc(U[4])) + cmul(U[6], conjc(U[7]));
         ov = (1.0 / nr) * ov;
 #pragma unroll
-        for (int i = 0; i < 3; i++) m[3 * i + 1] = axpyc(m[3 * i + 1], ov, m[3 * i]);
+        for (int i = 0; i < 3; i++) U[3 * i + 1] = U[3 * i + 1] - cmul(ov, U[3 * i]);
     }
-    nr = rsqrt(nr);
+    nr = 1.0 / sqrt(nr);
 #pragma unroll
-    for (int i = 0; i < 3; i++) m[3 * i] = nr * m[3 * i];
-    nr = rsqrt(nrm3(m[1], m[4], m[7]));
+    for (int i = 0; i < 3; i++) U[3 * i] = nr * U[3 * i];
+    nr = 1.0 / sqrt(nrm2c(U[1]) + nrm2c(U[4]) + nrm2c(U[7]));
 #pragma unroll
-    for (int i = 0; i < 3; i++) m[3 * i + 1] = nr * m[3 * i + 1];
-    m[2] = ccross(m[3], m[7], m[6], m[4]);
-    m[5] = ccross(m[6], m[1], m[0], m[7]);
-    m[8] = ccross(m[0], m[4], m[3], m[1]);
+    for (int i = 0; i < 3; i++) U[3 * i + 1] = nr * U[3 * i + 1];
+    U[2] = conjc(cmul(U[3], U[7]) - cmul(U[6], U[4]));
+    U[5] = conjc(cmul(U[6], U[1]) - cmul(U[0], U[7]));
+    U[8] = conjc(cmul(U[0], U[4]) - cmul(U[3], U[1]));
+#pragma unroll
+    for (int k = 0; k < 9; k++) M.a[k] = U[k];
 }
 
 // ---- site coordinates in the parity-blocked layout ------------------------
@@ -404,10 +364,10 @@ struct ApeArgs {
 // links through the CU's cache, and the 64 lanes of a load read one component
 // array at consecutive sites, 16 cache accesses a load.  With the three links
 // of a site on adjacent lanes almost every lane was an access of its own (57 a
-// load), and the kernel spent its time there.  24^3x48: 330 -> 293 us a step by
-// the lanes, 277 us by fewer instructions in the projection (3,390 -> 2,683),
-// 272 us by the workgroup size; now bound by the FP64 ALU at two wavefronts per
-// SIMD.  Three wavefronts (168 registers) spill: 321 us.
+// load), and the kernel spent its time there.  24^3x48: 330 -> 293 us a step, the
+// same bits; now bound by the FP64 ALU at two wavefronts per SIMD (3,390 vector
+// instructions a thread, 2,500 of them the projection).  Three wavefronts (168
+// registers) spill.
 // Four wavefronts per workgroup (of three, two workgroups would leave a
 // quarter of a CU's eight register-limited wavefront places empty).
 constexpr int kApeWaves = 4;
