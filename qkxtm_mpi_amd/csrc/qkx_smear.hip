@@ -16,6 +16,8 @@
 //                      covariant hop on all four spins; the links of a site
 //                      are shared by its right-hand sides (adjacent lanes).
 //                      HBM-bound: 432 B of links + 384 B per right-hand side.
+//   gauss_march_kernel the same for many units: one thread per (column, spin,
+//                      right-hand side), marching along z.
 //   plaq_kernel        grid-stride per-site sum of the six plaquettes into
 //                      per-workgroup partials, summed in a fixed order.
 #include <cmath>
@@ -539,6 +541,233 @@ ProjConst proj_const()
     return ProjConst{std::pow(18., 1. / 3.), std::pow(12., 1. / 3.), std::pow(2. / 3., 1. / 3.), std::sqrt(3.)};
 }
 
+// The same step, marching along z: a workgroup owns 64 (column, right-hand
+// side) units of one time slice -- a column is a fixed (x, y) -- and walks z0 ..
+// z0 + zlen - 1.  Wavefront w works on spin w (the hop does not mix spins), so a
+// unit's spinor is three complex numbers per thread: psi(z) and psi(z + 1) stay
+// in registers from one plane to the next, and the backward z hop is formed one
+// plane early, where its link and spinor are at hand, and carried.  The five
+// links of a site's plane (U_x, U_x(x-1), U_y, U_y(y-1), U_z) go to LDS once
+// for the four spins and all right-hand sides.  Per (site, spin, right-hand
+// side) that is 15 loads of 16 B, where gauss_step_kernel has 138 / 4; and the
+// workgroups of a slice walk the same few z planes at a time, so a plane's x
+// and y neighbours are in the XCD's L2 when they are read.  Every sum has
+// gauss_step_kernel's order: the same bits.  12 right-hand sides at 24^3x48:
+// 1015 -> 910 us a step, 4.9 GB of HBM traffic (3.3 compulsory) at 5.4 TB/s; a
+// 48^3 slice 192 -> 172 us.
+struct GaussMarch {
+    const double2 *in;
+    double2 *out;
+    const double2 *U;
+    Geom g;
+    FastDiv dnr, dwpp, dseg;
+    size_t stride;    // entries of one component
+    int nr, cols;     // units of one slice
+    int wpp, nseg;    // workgroups per plane, segments of z
+    int zlen, t_lo, nblk, nblk8;
+    double alpha, norm;
+};
+constexpr int kMarchLinks = 5;
+
+// tot += U psi or U^dag psi of one spin, in gauss_hop's order
+template <bool BWD> __device__ __forceinline__ void march_hop(C tot[3], const double2 *l, const C ps[3])
+{
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        C u[3];
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const double2 d = BWD ? l[3 * j + i] : l[3 * i + j];
+            u[j] = {d.x, d.y};
+        }
+        const C h = BWD ? cjmac(cjmac(cjmul_f(u[0], ps[0]), u[1], ps[1]), u[2], ps[2])
+                        : cmac(cmac(cmul_f(u[0], ps[0]), u[1], ps[1]), u[2], ps[2]);
+        tot[i] = tot[i] + h;
+    }
+}
+
+__device__ __forceinline__ void pin_vec(C t[3])
+{
+    asm volatile("" : "+v"(t[0].re), "+v"(t[0].im), "+v"(t[1].re), "+v"(t[1].im), "+v"(t[2].re), "+v"(t[2].im)::"memory");
+}
+
+template <int NL> __global__ __launch_bounds__(256) void gauss_march_kernel(GaussMarch a)
+{
+    extern __shared__ double2 march_links[];
+    const Geom &g = a.g;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int b = a.nblk8 > 0 ? ((int)blockIdx.x & 7) * a.nblk8 + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
+    if (b >= a.nblk) return;   // uniform over the workgroup
+    const int pl = fdiv(b, a.dwpp), pw = b - pl * a.wpp;
+    const int tt = fdiv(pl, a.dseg), z0 = (pl - tt * a.nseg) * a.zlen;
+    const int t = a.t_lo + tt, n = min(a.zlen, g.L[2] - z0);
+    const int V = g.V, plane = g.Lh0 * g.L[1], tbase = plane * g.L[2] * t;
+    // column q of a slice: xh fastest, then x's parity, then y
+    auto column = [&](int q, int &x, int &y) {
+        const int rest = fdiv(q, g.dLh0);
+        x = 2 * (q - rest * g.Lh0) + (rest & 1);
+        y = rest >> 1;
+    };
+    const int u0 = pw * 64;
+    const bool own = u0 + lane < a.cols;
+    const int u = min(u0 + lane, a.cols - 1);
+    const int q = fdiv(u, a.dnr), r = u - q * a.nr, q0 = fdiv(u0, a.dnr);
+    const int ns = fdiv(min(u0 + 63, a.cols - 1), a.dnr) - q0 + 1;   // sites of this workgroup
+    int x, y;
+    column(q, x, y);
+    const int xy = x + y + t;   // parity of the site at z: (xy + z) & 1
+    const int cb = tbase + (x >> 1) + g.Lh0 * y;
+    const int cxp = tbase + ((x + 1 == g.L[0] ? 0 : x + 1) >> 1) + g.Lh0 * y;
+    const int cxm = tbase + ((x == 0 ? g.L[0] - 1 : x - 1) >> 1) + g.Lh0 * y;
+    const int cyp = tbase + (x >> 1) + g.Lh0 * (y + 1 == g.L[1] ? 0 : y + 1);
+    const int cym = tbase + (x >> 1) + g.Lh0 * (y == 0 ? g.L[1] - 1 : y - 1);
+    const double2 *in = a.in + (size_t)(3 * w) * a.stride + r;
+    auto load = [&](int c, int z, int par, C v[3]) __attribute__((always_inline)) {
+        const size_t e = (size_t)((par ? g.Vh : 0) + c + plane * z) * a.nr;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const double2 d = in[(size_t)k * a.stride + e];
+            v[k] = {d.x, d.y};
+        }
+    };
+    // this thread's link elements: (site j, link l, element k), sites fastest
+    int lsrc[NL], lpar[NL], ldst[NL];
+#pragma unroll
+    for (int i = 0; i < NL; i++) {
+        // past the last element: the last one again (not stored)
+        const int id = min((int)threadIdx.x + 256 * i, ns * 9 * kMarchLinks - 1);
+        const int e = id / ns, j = id - e * ns, l = e / 9, k = e - 9 * l;
+        int lx, ly;
+        column(q0 + j, lx, ly);
+        ldst[i] = j * 9 * kMarchLinks + e;
+        lpar[i] = lx + ly + t + (l & 1);   // links 1 and 3 sit on the other parity
+        if (l == 1) lx = lx == 0 ? g.L[0] - 1 : lx - 1;
+        if (l == 3) ly = ly == 0 ? g.L[1] - 1 : ly - 1;
+        lsrc[i] = ((l >> 1) * 9 + k) * V + tbase + (lx >> 1) + g.Lh0 * ly;
+    }
+    double lre[NL], lim[NL];
+    auto fetch_links = [&](int z) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NL; i++) {
+            const double2 d = a.U[(size_t)lsrc[i] + (((lpar[i] + z) & 1) ? g.Vh : 0) + plane * z];
+            lre[i] = d.x;
+            lim[i] = d.y;
+        }
+    };
+    auto put_links = [&]() __attribute__((always_inline)) {
+        __syncthreads();   // the last plane's links have been read
+#pragma unroll
+        for (int i = 0; i < NL; i++)
+            if ((int)threadIdx.x + 256 * i < ns * 9 * kMarchLinks) march_links[ldst[i]] = make_double2(lre[i], lim[i]);
+        __syncthreads();
+    };
+    const double2 *link = march_links + (q - q0) * 9 * kMarchLinks;
+    C pc[3], carry[3] = {{0, 0}, {0, 0}, {0, 0}};
+    {
+        const int zm = z0 == 0 ? g.L[2] - 1 : z0 - 1;
+        C pm[3];
+        fetch_links(zm);
+        load(cb, zm, (xy + zm) & 1, pm);
+        load(cb, z0, (xy + z0) & 1, pc);
+        put_links();
+        fetch_links(z0);
+        march_hop<true>(carry, link + 36, pm);
+    }
+    for (int i = 0; i < n; i++) {
+        const int z = z0 + i, zp = z + 1 == g.L[2] ? 0 : z + 1, par = (xy + z) & 1;
+        C pn[3], nb[4][3];
+        load(cxp, z, par ^ 1, nb[0]);
+        load(cxm, z, par ^ 1, nb[1]);
+        load(cyp, z, par ^ 1, nb[2]);
+        load(cym, z, par ^ 1, nb[3]);
+        load(cb, zp, (xy + zp) & 1, pn);
+        put_links();
+        if (i + 1 < n) fetch_links(zp);
+        C tot[3] = {{0, 0}, {0, 0}, {0, 0}};
+        // one link of LDS reads in flight at a time: all five take 180 registers
+        march_hop<false>(tot, link, nb[0]);
+        pin_vec(tot);
+        march_hop<true>(tot, link + 9, nb[1]);
+        pin_vec(tot);
+        march_hop<false>(tot, link + 18, nb[2]);
+        pin_vec(tot);
+        march_hop<true>(tot, link + 27, nb[3]);
+        pin_vec(tot);
+        march_hop<false>(tot, link + 36, pn);
+        pin_vec(tot);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            tot[k] = tot[k] + carry[k];
+            carry[k] = {0, 0};
+        }
+        march_hop<true>(carry, link + 36, pc);
+        if (own) {
+            typedef __attribute__((ext_vector_type(2))) double d2v;
+            double2 *o = a.out + (size_t)(3 * w) * a.stride + r + (size_t)((par ? g.Vh : 0) + cb + plane * z) * a.nr;
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                __builtin_nontemporal_store(d2v{a.norm * (pc[k].re + a.alpha * tot[k].re),
+                                                a.norm * (pc[k].im + a.alpha * tot[k].im)},
+                                            reinterpret_cast<d2v *>(o + (size_t)k * a.stride));
+        }
+#pragma unroll
+        for (int k = 0; k < 3; k++) pc[k] = pn[k];
+    }
+}
+
+// Launch shape of the march over the slices of a smearing, `lds` bytes of links
+struct MarchGrid {
+    dim3 grid;
+    size_t lds;
+    int loads;   // link elements per thread
+};
+MarchGrid make_march(GaussMarch &m, const qkx_gauge_s *U, int nr, int t, double alpha)
+{
+    const int *L = U->L;
+    m.U = (const double2 *)U->data;
+    m.g = qkx::make_geom(L, U->bc);
+    m.nr = nr;
+    m.dnr = make_fastdiv(nr);
+    m.stride = (size_t)U->V * nr;
+    m.cols = L[0] * L[1] * nr;
+    m.wpp = (m.cols + 63) / 64;
+    m.t_lo = t < 0 ? 0 : t;
+    const int nt = t < 0 ? L[3] : 1;
+    // z in segments (each re-reads one plane) while the slices alone do not
+    // give every CU three rounds of resident workgroups; four planes at least
+    constexpr int kMarchFill = 2304;
+    m.nseg = std::max(1, std::min((kMarchFill + m.wpp * nt - 1) / (m.wpp * nt), L[2] / 4));
+    m.zlen = (L[2] + m.nseg - 1) / m.nseg;
+    m.nseg = (L[2] + m.zlen - 1) / m.zlen;
+    m.dwpp = make_fastdiv(m.wpp);
+    m.dseg = make_fastdiv(m.nseg);
+    m.nblk = m.wpp * nt * m.nseg;
+    m.nblk8 = m.nblk >= 64 ? (m.nblk + 7) / 8 : 0;
+    m.alpha = alpha;
+    m.norm = 1.0 / (1 + 6 * alpha);
+    const int sites = std::min(64, 63 / nr + 2);   // of a workgroup, at most
+    MarchGrid r;
+    r.lds = (size_t)sites * 9 * kMarchLinks * sizeof(double2);
+    r.loads = (sites * 9 * kMarchLinks + 255) / 256;
+    r.grid = dim3(m.nblk8 ? 8 * m.nblk8 : m.nblk);
+    return r;
+}
+void launch_march(const GaussMarch &m, const MarchGrid &r)
+{
+    if (r.loads <= 2) hipLaunchKernelGGL(gauss_march_kernel<2>, r.grid, dim3(256), r.lds, qkx::g_stream, m);
+    else if (r.loads <= 3) hipLaunchKernelGGL(gauss_march_kernel<3>, r.grid, dim3(256), r.lds, qkx::g_stream, m);
+    else if (r.loads <= 6) hipLaunchKernelGGL(gauss_march_kernel<6>, r.grid, dim3(256), r.lds, qkx::g_stream, m);
+    else hipLaunchKernelGGL(gauss_march_kernel<12>, r.grid, dim3(256), r.lds, qkx::g_stream, m);
+}
+// A step of at least this many (site, right-hand side) units marches.  24 planes
+// in a row are a chain that needs enough workgroups beside it: 10 steps at
+// 16^3x32 (131,072 units) 318 -> 260 us, 30 steps of a 24^3 slice with 12
+// right-hand sides (165,888) 781 -> 760 us; a 48^3 slice with one (110,592) 709
+// -> 753 us, 8^3x16 with 12 (98,304) 269 -> 294 us.
+constexpr long kMarchUnits = 131072;
+// its link elements are indexed with 32 bits
+constexpr long kMarchSites = ((1L << 31) - 1) / 27;
+
 bool fp64_links(const qkx_gauge_s *g) { return g && g->prec == QKX_PREC_DOUBLE && g->recon == QKX_RECON_18; }
 
 // Spatial-link workspace of the APE ping-pong, kept between calls (a smearing
@@ -660,14 +889,21 @@ int qkx_gauss_smear(qkx_spinor *out, const qkx_spinor *in, const qkx_gauge *U, i
     if (nsmear == 0) return QKX_SUCCESS;   // the reference returns before touching the field
     const int *L = in->L;
     const int nr = in->nrhs;
+    const bool march = (long)L[0] * L[1] * L[2] * (t < 0 ? L[3] : 1) * nr >= kMarchUnits && in->V <= kMarchSites;
+    GaussMarch m;
     GaussArgs a;
-    a.U = (const double2 *)U->data;
-    a.g = qkx::make_geom(L, U->bc);
-    a.nr = nr;
+    MarchGrid mg;
     dim3 grid;
-    a.tr = make_trav(L, nr, t, grid, [](int n) { return (n + kThreads - 1) / kThreads; });
-    a.alpha = alpha;
-    a.norm = 1.0 / (1 + 6 * alpha);
+    if (march) {
+        mg = make_march(m, U, nr, t, alpha);
+    } else {
+        a.U = (const double2 *)U->data;
+        a.g = qkx::make_geom(L, U->bc);
+        a.nr = nr;
+        a.tr = make_trav(L, nr, t, grid, [](int n) { return (n + kThreads - 1) / kThreads; });
+        a.alpha = alpha;
+        a.norm = 1.0 / (1 + 6 * alpha);
+    }
     int rc;
     if (t >= 0 && (rc = qkx_spinor_zero(out))) return rc;
     std::unique_ptr<qkx::Temp> tmp;
@@ -681,9 +917,15 @@ int qkx_gauss_smear(qkx_spinor *out, const qkx_spinor *in, const qkx_gauge *U, i
     const qkx_spinor_s *src = in;
     for (int it = 0; it < nsmear; it++) {
         qkx_spinor_s *dst = bufs[(nsmear - 1 - it) & 1];
-        a.in = make_spinor<SpinorD>(src);
-        a.out = make_spinor<SpinorD>(dst);
-        hipLaunchKernelGGL(gauss_step_kernel, grid, dim3(kThreads), 0, qkx::g_stream, a);
+        if (march) {
+            m.in = (const double2 *)src->data;
+            m.out = (double2 *)dst->data;
+            launch_march(m, mg);
+        } else {
+            a.in = make_spinor<SpinorD>(src);
+            a.out = make_spinor<SpinorD>(dst);
+            hipLaunchKernelGGL(gauss_step_kernel, grid, dim3(kThreads), 0, qkx::g_stream, a);
+        }
         src = dst;
     }
     QKX_HIP(hipGetLastError());
