@@ -64,24 +64,47 @@ int ensure_bstate(int nblocks)
     return QKX_SUCCESS;
 }
 
+// The workgroup's sum per right-hand side of v (thread g nr + r: group g of
+// `groups`, right-hand side r), compensated, by halving the groups in LDS; the
+// result is in threads r < nr.  A serial sum over the groups by those threads
+// is a chain of up to 85 dependent compensated additions: 4 of the 6 us that a
+// one-workgroup sum took.
+template <int T> __device__ __forceinline__ DD group_sum_rhs(DD v, int groups, int nr, double (&lh)[T], double (&ll)[T])
+{
+    const int t = threadIdx.x, g = t / nr;
+    lh[t] = v.hi;
+    ll[t] = v.lo;
+    __syncthreads();
+    for (int n = groups; n > 1;) {
+        const int h = (n + 1) >> 1;
+        if (g + h < n) {
+            v = dd_add(v, DD{lh[t + h * nr], ll[t + h * nr]});
+            lh[t] = v.hi;
+            ll[t] = v.lo;
+        }
+        __syncthreads();
+        n = h;
+    }
+    return v;
+}
+
 // sums[r] = sum_b part[b*nr + r] for r < nr, compensated (double-double), in
 // a fixed order; every thread of the workgroup sees the same values.
 __device__ void block_sums_rhs(const double *part, int nblocks, int nr, double *sums)
 {
+    if (nblocks == 1) {   // already summed
+        if ((int)threadIdx.x < nr) sums[threadIdx.x] = part[threadIdx.x];
+        __syncthreads();
+        return;
+    }
     __shared__ double lh[kT], ll[kT];
     const int groups = blockDim.x / nr;
     const int r = threadIdx.x % nr, g = threadIdx.x / nr;
     DD s{0.0, 0.0};
     if (g < groups)
         for (int b = g; b < nblocks; b += groups) s = dd_add(s, part[(size_t)b * nr + r]);
-    lh[threadIdx.x] = s.hi;
-    ll[threadIdx.x] = s.lo;
-    __syncthreads();
-    if ((int)threadIdx.x < nr) {
-        DD t{0.0, 0.0};
-        for (int gg = 0; gg < groups; gg++) t = dd_add(t, DD{lh[gg * nr + threadIdx.x], ll[gg * nr + threadIdx.x]});
-        sums[threadIdx.x] = dd_value(t);
-    }
+    s = group_sum_rhs(s, groups, nr, lh, ll);
+    if ((int)threadIdx.x < nr) sums[threadIdx.x] = dd_value(s);
     __syncthreads();
 }
 
@@ -156,6 +179,21 @@ __global__ __launch_bounds__(kT) void cgb_dir_kernel(S p, SR r, SX x, int n, int
     }
     __shared__ double r2n[NR], pap[NR];
     __shared__ int flag_s;
+    // this unit's p, r (and x) are requested before the sums and the decision,
+    // so their latency overlaps them
+    using T = typename SR::Real;
+    using TX = typename SX::Real;
+    const int u = blockIdx.x * blockDim.x + threadIdx.x;
+    const int rr = u % nr;
+    const bool xupd = HASX && mode == 0 && u < n;
+    typename S::Raw pw;
+    typename SR::Raw rw;
+    typename SX::Raw xw;
+    if (u < n) {
+        pw = p.template fetch<3>(u);
+        rw = r.template fetch<3>(u);
+        if (xupd) xw = x.template fetch<3>(u);
+    }
     block_sums_rhs(r2_part, nr2, nr, r2n);
     if (mode == 0) block_sums_rhs(pap_part, npap, nr, pap);
     if (threadIdx.x == 0) {
@@ -177,16 +215,12 @@ __global__ __launch_bounds__(kT) void cgb_dir_kernel(S p, SR r, SX x, int n, int
     }
     __syncthreads();
     const int flag = flag_s;
-    const int u = blockIdx.x * blockDim.x + threadIdx.x;
-    const int rr = u % nr;
     Cx<typename S::Real> pv[12];
-    const bool xupd = HASX && mode == 0 && u < n;
+    if (u < n) p.template unpack<3>(pw, pv);
     if (xupd) {
-        using TX = typename SX::Real;
         const TX ax = TX(frozen(cur, rr) ? 0.0 : cur->r2[rr] / pap[rr]);
         Cx<TX> xv[12];
-        x.load(u, xv);
-        p.load(u, pv);
+        x.template unpack<3>(xw, xv);
 #pragma unroll
         for (int k = 0; k < 12; k++) xv[k] = {xv[k].re + ax * TX(pv[k].re), xv[k].im + ax * TX(pv[k].im)};
         x.store(u, xv);
@@ -211,11 +245,9 @@ __global__ __launch_bounds__(kT) void cgb_dir_kernel(S p, SR r, SX x, int n, int
     double beta;
     if (mode == 0) beta = frozen(cur, rr) ? 0.0 : r2n[rr] / cur->r2[rr];
     else beta = cur->r2_old[rr] > 0 ? r2n[rr] / cur->r2_old[rr] : 0.0;
-    using T = typename SR::Real;
     const T b = T(beta);
     Cx<T> rv[12];
-    if (!xupd) p.load(u, pv);
-    r.load(u, rv);
+    r.template unpack<3>(rw, rv);
     Cx<typename S::Real> out[12];
 #pragma unroll
     for (int k = 0; k < 12; k++)
@@ -252,14 +284,8 @@ __global__ __launch_bounds__(1024) void sum_rhs_kernel(const double *part, int n
             const size_t i = (size_t)b * nr + r;
             v = dd_in ? dd_add(v, DD{part[2 * i], part[2 * i + 1]}) : dd_add(v, part[i]);
         }
-    lh[threadIdx.x] = v.hi;
-    ll[threadIdx.x] = v.lo;
-    __syncthreads();
-    if ((int)threadIdx.x < nr) {
-        DD t{0.0, 0.0};
-        for (int gg = 0; gg < groups; gg++) t = dd_add(t, DD{lh[gg * nr + threadIdx.x], ll[gg * nr + threadIdx.x]});
-        out[threadIdx.x] = dd_value(t);
-    }
+    v = group_sum_rhs(v, groups, nr, lh, ll);
+    if ((int)threadIdx.x < nr) out[threadIdx.x] = dd_value(v);
 }
 
 // First stage of a many-row sum: workgroup g sums rows [g chunk, (g+1) chunk)
@@ -275,15 +301,11 @@ __global__ __launch_bounds__(kT) void sum_rhs_chunks_kernel(const double *part, 
     DD v{0.0, 0.0};
     if (g < groups)
         for (int b = b0 + g; b < b1; b += groups) v = dd_add(v, part[(size_t)b * nr + r]);
-    lh[threadIdx.x] = v.hi;
-    ll[threadIdx.x] = v.lo;
-    __syncthreads();
+    v = group_sum_rhs(v, groups, nr, lh, ll);
     if ((int)threadIdx.x < nr) {
-        DD t{0.0, 0.0};
-        for (int gg = 0; gg < groups; gg++) t = dd_add(t, DD{lh[gg * nr + threadIdx.x], ll[gg * nr + threadIdx.x]});
         const size_t i = (size_t)blockIdx.x * nr + threadIdx.x;
-        out[2 * i] = t.hi;
-        out[2 * i + 1] = t.lo;
+        out[2 * i] = v.hi;
+        out[2 * i + 1] = v.lo;
     }
 }
 
