@@ -711,7 +711,7 @@ def run_smear(q, args):
                                "(whole lattice)", "lattice": list(L)},
         "roofline": {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": gbs / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": "gauss_step_kernel, whole lattice, 12 right-hand sides",
+                     "kernel": "gauss_march_kernel, whole lattice, 12 right-hand sides",
                      "avg_launch_us": us_gf, "bytes_per_launch": by_gf,
                      "timing": "HIP events around 11 and 1 smearing steps, difference / 10, median of 3"},
         "kernels": {"ape_step_us": us_ape, "ape_step_GBs": by_ape / (us_ape * 1e-6) / 1e9,

@@ -128,7 +128,9 @@ int  qkx_set_tuning(int xcd_remap, int block, int depth64, int depth32);
  * -- x, then blocks of up to 8 y rows and up to 8 t slices, then z -- so that
  * neighbour spinors and backward links are reused from L2; 0: checkerboard
  * index order; 2 (default): blocked for the full-lattice FP64 hops (tm and
- * its family, the full-lattice CG), checkerboard order for the rest.  Results
+ * its family, the full-lattice CG) and for batches of 8 or more right-hand
+ * sides whose time slice exceeds an XCD's 4 MB L2, checkerboard order for the
+ * rest.  Results
  * per site are identical; reductions sum in another order. */
 int  qkx_set_site_order(int blocked);
 /* Single-RHS FP16 hops on one parity (FP16 12-real links, checkerboard site

@@ -755,7 +755,7 @@ def set_batch_link_sharing(mode=1):
 def set_site_order(mode=2):
     """Site order of the hopping kernels: 1 (or True) blocked, 0 (or False)
     checkerboard index order, 2 (default) blocked for the full-lattice FP64
-    hops only."""
+    hops and for batches of 8 or more whose time slice exceeds 4 MB."""
     _check(lib().qkx_set_site_order(int(mode)), "qkx_set_site_order")
 
 

@@ -71,7 +71,7 @@ __global__ void eo_weights_kernel(const float2 *w, const uint32_t *wb, int bf, i
 // order the t neighbours' 1.2 KB per site (12 RHS) leave the L2 before they
 // come round, and the two kernels fetched 0.92 and 2.06 GB, now 0.62 and 1.65.
 // 12 RHS, FP16, CH = 4, 24^3x48, forward and adjoint: 1979 us with the mixing on
-// the vector ALU, 1530 us on the matrix cores, 1491 us in blocks; now bound
+// the vector ALU, 1491-1531 us on the matrix cores, walked in blocks; now bound
 // by the vector and matrix pipes (1,680 vector instructions, 400 MFMAs a thread).
 struct EoArgs {
     Geom g;
