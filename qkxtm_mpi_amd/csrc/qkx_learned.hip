@@ -465,6 +465,9 @@ void grad_grid(int ch, int V, int &bs, int &nb)
 int net_buffers(qkx_net_s *n, const int L[4])
 {
     if (n->fh && n->L[0] == L[0] && n->L[1] == L[1] && n->L[2] == L[2] && n->L[3] == L[3]) return QKX_SUCCESS;
+    // no lattice until every buffer is there: after a failed allocation the next
+    // call starts over
+    for (int d = 0; d < 4; d++) n->L[d] = 0;
     float4 **bufs[3] = {&n->fh, &n->gout, &n->gh};
     for (auto b : bufs) {
         if (*b) (void)hipFree(*b);
@@ -473,7 +476,6 @@ int net_buffers(qkx_net_s *n, const int L[4])
     const size_t V = (size_t)L[0] * L[1] * L[2] * L[3];
     const int chans[3] = {n->ch, 4, n->ch};
     for (int i = 0; i < 3; i++) QKX_HIP(hipMalloc(bufs[i], sizeof(float2) * 3 * chans[i] * V));
-    for (int d = 0; d < 4; d++) n->L[d] = L[d];
     // partials: both layers' gradients, then the loss
     int bs, nb;
     grad_grid(n->ch, (int)V, bs, nb);
@@ -485,6 +487,7 @@ int net_buffers(qkx_net_s *n, const int L[4])
         QKX_HIP(hipMalloc(&n->part, sizeof(double) * need));
         n->part_cap = need;
     }
+    for (int d = 0; d < 4; d++) n->L[d] = L[d];
     return QKX_SUCCESS;
 }
 
