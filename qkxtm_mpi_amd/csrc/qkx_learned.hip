@@ -295,10 +295,21 @@ __device__ __forceinline__ void wgrad_hold(const S &v, const GaugeF18 &U, const 
     wgrad_step();
     if constexpr (P + 1 < P1) wgrad_hold<P + 1, P1>(v, U, g, n, live, next, t + 1, f, fr);
 }
+// LDS of a workgroup, one buffer for whichever path group it takes (a static one
+// in wgrad_group would be there once per group: 78 KB for 17 at CH = 16, and two
+// workgroups to a CU where the launch counts on eight of 64 threads): a row of the
+// group's FP32 sums per 16 lanes, padded so that the rows start on different banks.
+extern __shared__ float wgrad_lds[];
+constexpr int wgrad_numbers(int ch, int np) { return np * 4 * ch * 2; }
+constexpr int wgrad_row(int numbers) { return numbers + 4; }
+inline size_t wgrad_lds_bytes(int ch, int np, int bs)
+{
+    return (size_t)(bs / 16) * wgrad_row(wgrad_numbers(ch, np)) * sizeof(float);
+}
 template <int CH, int P0, int NP, class S>
 __device__ __forceinline__ void wgrad_group(const Hid &f, const S &v, const GaugeF18 &U, const Geom &g, double *part)
 {
-    constexpr int H = CH / 4;
+    constexpr int H = CH / 4, W = wgrad_numbers(CH, NP);
     f4v zr[NP][H], zi[NP][H];
 #pragma unroll
     for (int p = 0; p < NP; p++)
@@ -334,7 +345,6 @@ __device__ __forceinline__ void wgrad_group(const Hid &f, const S &v, const Gaug
         }
     }
     // sums of 16 lanes' blocks in registers, of the workgroup's 16-lane rows in LDS and FP64
-    __shared__ float red[NP * H * 8 * 4][kT / 16 + 1];
     const int row = threadIdx.x >> 4, rows = blockDim.x >> 4;
 #pragma unroll
     for (int p = 0; p < NP; p++)
@@ -346,6 +356,7 @@ __device__ __forceinline__ void wgrad_group(const Hid &f, const S &v, const Gaug
                 zi[p][h][k] = row_sum(zi[p][h][k]);
             }
     if ((threadIdx.x & 12) == 0) {
+        float *dst = wgrad_lds + row * wgrad_row(W);
 #pragma unroll
         for (int p = 0; p < NP; p++)
 #pragma unroll
@@ -353,14 +364,15 @@ __device__ __forceinline__ void wgrad_group(const Hid &f, const S &v, const Gaug
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     const int w = (p * 4 + i) * CH + 4 * h + k;   // row k: channel of f, column i: vector of v
-                    red[2 * w][row] = zr[p][h][k];
-                    red[2 * w + 1][row] = zi[p][h][k];
+                    dst[2 * w] = zr[p][h][k];
+                    dst[2 * w + 1] = zi[p][h][k];
                 }
     }
     __syncthreads();
-    for (int w = threadIdx.x; w < NP * 4 * CH * 2; w += blockDim.x) {
+    for (int w = threadIdx.x; w < W; w += blockDim.x) {
         double t = 0;
-        for (int q = 0; q < rows; q++) t += (double)red[w][q];
+#pragma unroll 4
+        for (int q = 0; q < rows; q++) t += (double)wgrad_lds[q * wgrad_row(W) + w];
         part[(size_t)(P0 * 4 * CH * 2 + w) * gridDim.x + blockIdx.x] = t;
     }
 }
@@ -579,8 +591,8 @@ int launch_wgrad(qkx_net_s *n, Hid f, const qkx_spinor_s *v, const qkx_gauge_s *
     return with_ch(n, [&](auto CHC) {
         constexpr int CH = decltype(CHC)::value;
         auto go = [&](auto S) {
-            hipLaunchKernelGGL((net_wgrad_kernel<CH, decltype(S)>), dim3(nb, wgrad_groups(CH)), dim3(bs), 0,
-                               qkx::g_stream, f, S, G, g, part);
+            hipLaunchKernelGGL((net_wgrad_kernel<CH, decltype(S)>), dim3(nb, wgrad_groups(CH)), dim3(bs),
+                               wgrad_lds_bytes(CH, wgrad_np(CH), bs), qkx::g_stream, f, S, G, g, part);
             QKX_HIP(hipGetLastError());
             return QKX_SUCCESS;
         };

@@ -54,3 +54,11 @@ def test_batched_direction_step_occupancy(kernels):
     """Four wavefronts per SIMD at least: 128 of its 512 registers."""
     for n, k in named(kernels, "cgb_dir_kernel").items():
         assert k["vgpr_count"] <= 128 and k["vgpr_spill_count"] == 0, (n, k)
+
+
+def test_weight_gradient_lds(kernels):
+    """One sum buffer for all path groups, sized by the launch: nothing static, so
+    that the eight 64-thread workgroups which the launch rule counts on per CU
+    (160 KB of LDS) are resident whatever the hidden channels."""
+    for n, k in named(kernels, "net_wgrad_kernel").items():
+        assert k["group_segment_fixed_size"] * 8 <= 160 * 1024, (n, k)
