@@ -60,10 +60,18 @@ __device__ __forceinline__ NetSite layer_site(const Geom &g, int nblk8, bool &ow
     return net_site(g, p, s - p * g.Vh);
 }
 
-// Full-lattice layer 4 -> CH (or the adjoint of a layer CH -> 4).
+// An FP64 field to be rounded into an FP32 one beside other work, or nothing
+// (from.p null).
+struct RoundOff {
+    SpinorD from;
+    SpinorF to;
+};
+
+// Full-lattice layer 4 -> CH (or the adjoint of a layer CH -> 4, which takes a
+// RoundOff along in a wavefront that is done).
 template <int CH, bool ADJ, bool BF, class S>
 __global__ __launch_bounds__(kLayerT) QKX_NET_REGS void net_expand_kernel(S in, Hid out, GaugeF18 U, Geom g, int nblk8,
-                                                                          LayerWeights<4, CH, ADJ, BF> wt)
+                                                                          LayerWeights<4, CH, ADJ, BF> wt, RoundOff ro)
 {
     constexpr int H = CH / 4;
     __shared__ f4v part[2][H * 6][64];
@@ -92,6 +100,16 @@ __global__ __launch_bounds__(kLayerT) QKX_NET_REGS void net_expand_kernel(S in, 
             }
     }
     __syncthreads();
+    if constexpr (ADJ) {
+        if (w == 1 && own && ro.from.p) {
+            Cx<double> d[12];
+            Cx<float> f[12];
+            ro.from.load(n.s, d);
+#pragma unroll
+            for (int k = 0; k < 12; k++) f[k] = {(float)d[k].re, (float)d[k].im};
+            ro.to.store(n.s, f);
+        }
+    }
     if (w > 0) return;
 #pragma unroll
     for (int h = 0; h < H; h++)
@@ -223,20 +241,20 @@ __device__ __forceinline__ void quad_vectors(Cx<float> v[12], bool live)
     }
 }
 // the operands of one path
-template <class S> struct GradOps {
-    typename S::Raw psi;
+struct GradOps {
+    SpinorF::Raw psi;
     GaugeF18::Raw link;
 };
-template <int P, class S>
-__device__ __forceinline__ void wgrad_fetch(const S &v, const GaugeF18 &U, const Geom &g, const NetSite &n, GradOps<S> &o)
+template <int P>
+__device__ __forceinline__ void wgrad_fetch(const SpinorF &v, const GaugeF18 &U, const Geom &g, const NetSite &n, GradOps &o)
 {
     o.psi = v.template fetch<3>(path_site<P>(n));
     if constexpr (P > 0) o.link = LinkGlobal{U, g, n}.template fetch<P>();
 }
 // t = T_P v of the lane's site, as quad_vectors leaves it
-template <int P, class S>
-__device__ __forceinline__ void wgrad_transport(const S &v, const GaugeF18 &U, const Geom &g, const NetSite &n, bool live,
-                                                const GradOps<S> &o, Cx<float> t[12])
+template <int P>
+__device__ __forceinline__ void wgrad_transport(const SpinorF &v, const GaugeF18 &U, const Geom &g, const NetSite &n,
+                                                bool live, const GradOps &o, Cx<float> t[12])
 {
     Cx<float> x[12];
     (void)unpack_spinor(v, o.psi, x);
@@ -271,11 +289,11 @@ __device__ __forceinline__ void wgrad_tiles(const Cx<float> f[12], const Cx<floa
     }
 }
 // one tile per path (CH = 4): f stays, the transports come one at a time
-template <int P, int P1, class S>
-__device__ __forceinline__ void wgrad_each(const S &v, const GaugeF18 &U, const Geom &g, const NetSite &n, bool live,
-                                           const GradOps<S> &o, const Cx<float> f[12], f4v (*zr)[1], f4v (*zi)[1])
+template <int P, int P1>
+__device__ __forceinline__ void wgrad_each(const SpinorF &v, const GaugeF18 &U, const Geom &g, const NetSite &n, bool live,
+                                           const GradOps &o, const Cx<float> f[12], f4v (*zr)[1], f4v (*zi)[1])
 {
-    GradOps<S> next;
+    GradOps next;
     if constexpr (P + 1 < P1) wgrad_fetch<P + 1>(v, U, g, n, next);
     Cx<float> t[1][12];
     wgrad_transport<P>(v, U, g, n, live, o, t[0]);
@@ -284,11 +302,11 @@ __device__ __forceinline__ void wgrad_each(const S &v, const GaugeF18 &U, const 
     if constexpr (P + 1 < P1) wgrad_each<P + 1, P1>(v, U, g, n, live, next, f, zr + 1, zi + 1);
 }
 // the transports of paths P .. P1 - 1, and f's first channels requested
-template <int P, int P1, class S>
-__device__ __forceinline__ void wgrad_hold(const S &v, const GaugeF18 &U, const Geom &g, const NetSite &n, bool live,
-                                           const GradOps<S> &o, Cx<float> (*t)[12], const Hid &f, Hid::Raw &fr)
+template <int P, int P1>
+__device__ __forceinline__ void wgrad_hold(const SpinorF &v, const GaugeF18 &U, const Geom &g, const NetSite &n, bool live,
+                                           const GradOps &o, Cx<float> (*t)[12], const Hid &f, Hid::Raw &fr)
 {
-    GradOps<S> next;
+    GradOps next;
     if constexpr (P + 1 < P1) wgrad_fetch<P + 1>(v, U, g, n, next);
     else fr = f.fetch(0, n.s);
     wgrad_transport<P>(v, U, g, n, live, o, *t);
@@ -306,8 +324,8 @@ inline size_t wgrad_lds_bytes(int ch, int np, int bs)
 {
     return (size_t)(bs / 16) * wgrad_row(wgrad_numbers(ch, np)) * sizeof(float);
 }
-template <int CH, int P0, int NP, class S>
-__device__ __forceinline__ void wgrad_group(const Hid &f, const S &v, const GaugeF18 &U, const Geom &g, double *part)
+template <int CH, int P0, int NP>
+__device__ __forceinline__ void wgrad_group(const Hid &f, const SpinorF &v, const GaugeF18 &U, const Geom &g, double *part)
 {
     constexpr int H = CH / 4, W = wgrad_numbers(CH, NP);
     f4v zr[NP][H], zi[NP][H];
@@ -324,7 +342,7 @@ __device__ __forceinline__ void wgrad_group(const Hid &f, const S &v, const Gaug
         const int p = s >= g.Vh ? 1 : 0;
         const NetSite n = net_site(g, p, s - p * g.Vh);
         Cx<float> ff[12];
-        GradOps<S> o0;
+        GradOps o0;
         wgrad_fetch<P0>(v, U, g, n, o0);
         if constexpr (H == 1) {
             Hid::unpack(f.fetch(0, s), ff);
@@ -377,19 +395,20 @@ __device__ __forceinline__ void wgrad_group(const Hid &f, const S &v, const Gaug
     }
 }
 // paths per group: the sums take 2 CH registers per path, the transports held
-// beside them 24; one more path per group spills (CH = 16: 83 us with three)
+// beside them 24; one more path per group spills (CH = 16: 83 us with three), and
+// so does an FP64 v (134 registers at CH = 8), which is therefore rounded first
 constexpr int wgrad_np(int ch) { return ch == 4 ? 9 : ch == 8 ? 3 : 2; }
 constexpr int wgrad_groups(int ch) { return (9 + wgrad_np(ch) - 1) / wgrad_np(ch); }
-template <int CH, int G, class S>
-__device__ __forceinline__ void wgrad_select(const Hid &f, const S &v, const GaugeF18 &U, const Geom &g, double *part)
+template <int CH, int G>
+__device__ __forceinline__ void wgrad_select(const Hid &f, const SpinorF &v, const GaugeF18 &U, const Geom &g, double *part)
 {
     constexpr int P0 = G * wgrad_np(CH), NP = P0 + wgrad_np(CH) <= 9 ? wgrad_np(CH) : 9 - P0;
     if constexpr (G + 1 == wgrad_groups(CH)) wgrad_group<CH, P0, NP>(f, v, U, g, part);
     else if ((int)blockIdx.y == G) wgrad_group<CH, P0, NP>(f, v, U, g, part);
     else wgrad_select<CH, G + 1>(f, v, U, g, part);
 }
-template <int CH, class S>
-__global__ __launch_bounds__(kT) QKX_NET_REGS void net_wgrad_kernel(Hid f, S v, GaugeF18 U, Geom g, double *part)
+template <int CH>
+__global__ __launch_bounds__(kT) QKX_NET_REGS void net_wgrad_kernel(Hid f, SpinorF v, GaugeF18 U, Geom g, double *part)
 {
     wgrad_select<CH, 0>(f, v, U, g, part);
 }
@@ -527,7 +546,9 @@ template <class F> int with_bf(const qkx_net_s *n, F fn)
 Hid hid_of(float4 *p, int V) { return Hid{p, (size_t)V}; }
 
 // layer 1 of a spinor, or (ADJ) the adjoint of layer 2, into a hidden field
-template <bool ADJ> int launch_expand(qkx_net_s *n, const qkx_spinor_s *in, const SpinorF *inf, Hid out, const qkx_gauge_s *U)
+template <bool ADJ>
+int launch_expand(qkx_net_s *n, const qkx_spinor_s *in, const SpinorF *inf, Hid out, const qkx_gauge_s *U,
+                  const RoundOff &ro = RoundOff{})
 {
     const Geom g = qkx::make_geom(U->L, U->bc);
     const GaugeF18 G = make_gauge<GaugeF18>(U);
@@ -541,7 +562,7 @@ template <bool ADJ> int launch_expand(qkx_net_s *n, const qkx_spinor_s *in, cons
             const LayerWeights<4, CH, ADJ, BF> w{BF ? (const void *)(n->wb + off) : (const void *)(n->w + off)};
             auto go = [&](auto S) {
                 hipLaunchKernelGGL((net_expand_kernel<CH, ADJ, BF, decltype(S)>), dim3(nb), dim3(kLayerT), 0,
-                                   qkx::g_stream, S, out, G, g, nblk8, w);
+                                   qkx::g_stream, S, out, G, g, nblk8, w, ro);
                 QKX_HIP(hipGetLastError());
                 return QKX_SUCCESS;
             };
@@ -583,21 +604,17 @@ int launch_contract(qkx_net_s *n, qkx_spinor_s *out, const qkx_spinor_s *e, cons
     });
 }
 
-// Z of a hidden field and a spinor (v) or the loss gradient (v null)
-int launch_wgrad(qkx_net_s *n, Hid f, const qkx_spinor_s *v, const qkx_gauge_s *U, double *part, int bs, int nb)
+// Z of a hidden field f and a spinor v
+int launch_wgrad(qkx_net_s *n, Hid f, SpinorF v, const qkx_gauge_s *U, double *part, int bs, int nb)
 {
     const Geom g = qkx::make_geom(U->L, U->bc);
     const GaugeF18 G = make_gauge<GaugeF18>(U);
     return with_ch(n, [&](auto CHC) {
         constexpr int CH = decltype(CHC)::value;
-        auto go = [&](auto S) {
-            hipLaunchKernelGGL((net_wgrad_kernel<CH, decltype(S)>), dim3(nb, wgrad_groups(CH)), dim3(bs),
-                               wgrad_lds_bytes(CH, wgrad_np(CH), bs), qkx::g_stream, f, S, G, g, part);
-            QKX_HIP(hipGetLastError());
-            return QKX_SUCCESS;
-        };
-        if (v) return with_spinor(v, go);
-        return go(SpinorF{n->gout, g.V});
+        hipLaunchKernelGGL(net_wgrad_kernel<CH>, dim3(nb, wgrad_groups(CH)), dim3(bs),
+                           wgrad_lds_bytes(CH, wgrad_np(CH), bs), qkx::g_stream, f, v, G, g, part);
+        QKX_HIP(hipGetLastError());
+        return QKX_SUCCESS;
     });
 }
 
@@ -748,9 +765,14 @@ int qkx_net_accumulate_grad(qkx_net *n, const qkx_spinor *r, const qkx_spinor *e
     const SpinorF gout{n->gout, V};
     if ((rc = launch_expand<false>(n, r, nullptr, fh, U))) return rc;
     if ((rc = launch_contract(n, nullptr, e, U, lpart))) return rc;
-    if ((rc = launch_wgrad(n, fh, nullptr, U, z2, bs, nb))) return rc;
-    if ((rc = launch_expand<true>(n, nullptr, &gout, gh, U))) return rc;
-    if ((rc = launch_wgrad(n, gh, r, U, z1, bs, nb))) return rc;
+    if ((rc = launch_wgrad(n, fh, gout, U, z2, bs, nb))) return rc;
+    // layer 1's gradient gathers r nine times: an FP64 one is rounded once, into
+    // the hidden channels of the forward pass, which nothing reads any more
+    const SpinorF rf{n->fh, V};
+    const bool r64 = r->prec == QKX_PREC_DOUBLE;
+    const RoundOff ro{r64 ? make_spinor<SpinorD>(r) : SpinorD{}, rf};
+    if ((rc = launch_expand<true>(n, nullptr, &gout, gh, U, ro))) return rc;
+    if ((rc = launch_wgrad(n, gh, r64 ? rf : make_spinor<SpinorF>(r), U, z1, bs, nb))) return rc;
     hipLaunchKernelGGL(grad_finish_kernel, dim3(2 * 9 * 4 * n->ch + 1), dim3(64), 0, qkx::g_stream, z1, z2, nb, lpart,
                        loss_blocks(V), n->ch, n->grad, n->loss);
     QKX_HIP(hipGetLastError());

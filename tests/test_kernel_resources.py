@@ -62,3 +62,10 @@ def test_weight_gradient_lds(kernels):
     (160 KB of LDS) are resident whatever the hidden channels."""
     for n, k in named(kernels, "net_wgrad_kernel").items():
         assert k["group_segment_fixed_size"] * 8 <= 160 * 1024, (n, k)
+
+
+def test_learned_kernels_do_not_spill(kernels):
+    """The network's layers and gradients keep their sums in registers."""
+    for part in ("net_wgrad_kernel", "net_expand_kernel", "net_contract_kernel", "eo_hidden_kernel", "eo_out_kernel"):
+        for n, k in named(kernels, part).items():
+            assert k["vgpr_spill_count"] == 0, (n, k)
