@@ -313,86 +313,104 @@ __device__ __forceinline__ void wgrad_hold(const SpinorF &v, const GaugeF18 &U, 
     wgrad_step();
     if constexpr (P + 1 < P1) wgrad_hold<P + 1, P1>(v, U, g, n, live, next, t + 1, f, fr);
 }
+// The sums of a workgroup's lanes are FP32 over kGradFlush rounds of its sites at
+// most (192 products), then go to FP64 in LDS: without that their length, and
+// with it their rounding, grows with the volume.  24^3x48, CH = 8 (16 rounds):
+// 801 us without, 832, 822, 818 and 806 after every 1, 2, 4 and 8 rounds.
+constexpr int kGradFlush = 8;
 // LDS of a workgroup, one buffer for whichever path group it takes (a static one
 // in wgrad_group would be there once per group: 78 KB for 17 at CH = 16, and two
-// workgroups to a CU where the launch counts on eight of 64 threads): a row of the
-// group's FP32 sums per 16 lanes, padded so that the rows start on different banks.
-extern __shared__ float wgrad_lds[];
+// workgroups to a CU where the launch counts on eight of 64 threads): the FP64
+// sums of the group's numbers, then a row of their FP32 sums per 16 lanes, padded
+// so that the rows start on different banks.
+extern __shared__ double wgrad_lds[];
 constexpr int wgrad_numbers(int ch, int np) { return np * 4 * ch * 2; }
 constexpr int wgrad_row(int numbers) { return numbers + 4; }
 inline size_t wgrad_lds_bytes(int ch, int np, int bs)
 {
-    return (size_t)(bs / 16) * wgrad_row(wgrad_numbers(ch, np)) * sizeof(float);
+    const int w = wgrad_numbers(ch, np);
+    return w * sizeof(double) + (size_t)(bs / 16) * wgrad_row(w) * sizeof(float);
 }
 template <int CH, int P0, int NP>
 __device__ __forceinline__ void wgrad_group(const Hid &f, const SpinorF &v, const GaugeF18 &U, const Geom &g, double *part)
 {
     constexpr int H = CH / 4, W = wgrad_numbers(CH, NP);
-    f4v zr[NP][H], zi[NP][H];
-#pragma unroll
-    for (int p = 0; p < NP; p++)
-#pragma unroll
-        for (int h = 0; h < H; h++) zr[p][h] = zi[p][h] = f4v{0.f, 0.f, 0.f, 0.f};
-    const int i = threadIdx.x & 3;
+    double *tot = wgrad_lds;   // each number by its own thread
+    float *red = reinterpret_cast<float *>(tot + W);
+    const int step = gridDim.x * blockDim.x;
+    for (int w = threadIdx.x; w < W; w += blockDim.x) tot[w] = 0;
     // the same number of rounds in every wavefront of the workgroup
-    for (int s0 = blockIdx.x * blockDim.x; s0 < g.V; s0 += gridDim.x * blockDim.x) {
-        const int s1 = s0 + (int)threadIdx.x;
-        const bool live = s1 < g.V;
-        const int s = min(s1, g.V - 1);
-        const int p = s >= g.Vh ? 1 : 0;
-        const NetSite n = net_site(g, p, s - p * g.Vh);
-        Cx<float> ff[12];
-        GradOps o0;
-        wgrad_fetch<P0>(v, U, g, n, o0);
-        if constexpr (H == 1) {
-            Hid::unpack(f.fetch(0, s), ff);
-            quad_vectors(ff, live);
-            wgrad_each<P0, P0 + NP>(v, U, g, n, live, o0, ff, zr, zi);
-        } else {   // the transports stay, the channels come four at a time
-            Cx<float> t[NP][12];
-            Hid::Raw fr;
-            wgrad_hold<P0, P0 + NP>(v, U, g, n, live, o0, t, f, fr);
+    for (int s0 = blockIdx.x * blockDim.x; s0 < g.V;) {
+        f4v zr[NP][H], zi[NP][H];
 #pragma unroll
-            for (int h = 0; h < H; h++) {
-                Hid::unpack(fr, ff);
-                if (h + 1 < H) fr = f.fetch(h + 1, s);
+        for (int p = 0; p < NP; p++)
+#pragma unroll
+            for (int h = 0; h < H; h++) zr[p][h] = zi[p][h] = f4v{0.f, 0.f, 0.f, 0.f};
+        for (int k = 0; k < kGradFlush && s0 < g.V; k++, s0 += step) {
+            const int s1 = s0 + (int)threadIdx.x;
+            const bool live = s1 < g.V;
+            const int s = min(s1, g.V - 1);
+            const int p = s >= g.Vh ? 1 : 0;
+            const NetSite n = net_site(g, p, s - p * g.Vh);
+            Cx<float> ff[12];
+            GradOps o0;
+            wgrad_fetch<P0>(v, U, g, n, o0);
+            if constexpr (H == 1) {
+                Hid::unpack(f.fetch(0, s), ff);
                 quad_vectors(ff, live);
-                wgrad_tiles<NP>(ff, t, &zr[0][h], &zi[0][h], H);
-                wgrad_step();
+                wgrad_each<P0, P0 + NP>(v, U, g, n, live, o0, ff, zr, zi);
+            } else {   // the transports stay, the channels come four at a time
+                Cx<float> t[NP][12];
+                Hid::Raw fr;
+                wgrad_hold<P0, P0 + NP>(v, U, g, n, live, o0, t, f, fr);
+#pragma unroll
+                for (int h = 0; h < H; h++) {
+                    Hid::unpack(fr, ff);
+                    if (h + 1 < H) fr = f.fetch(h + 1, s);
+                    quad_vectors(ff, live);
+                    wgrad_tiles<NP>(ff, t, &zr[0][h], &zi[0][h], H);
+                    wgrad_step();
+                }
             }
         }
-    }
-    // sums of 16 lanes' blocks in registers, of the workgroup's 16-lane rows in LDS and FP64
-    const int row = threadIdx.x >> 4, rows = blockDim.x >> 4;
-#pragma unroll
-    for (int p = 0; p < NP; p++)
-#pragma unroll
-        for (int h = 0; h < H; h++)
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                zr[p][h][k] = row_sum(zr[p][h][k]);
-                zi[p][h][k] = row_sum(zi[p][h][k]);
-            }
-    if ((threadIdx.x & 12) == 0) {
-        float *dst = wgrad_lds + row * wgrad_row(W);
+        // sums of 16 lanes' blocks in registers, of the workgroup's 16-lane rows in
+        // FP64.  The lane is opaque here: the addresses formed from it would
+        // otherwise be kept in registers over the rounds.
+        int lane = threadIdx.x;
+        asm volatile("" : "+v"(lane));
+        const int i = lane & 3, row = lane >> 4, rows = blockDim.x >> 4;
 #pragma unroll
         for (int p = 0; p < NP; p++)
 #pragma unroll
             for (int h = 0; h < H; h++)
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
-                    const int w = (p * 4 + i) * CH + 4 * h + k;   // row k: channel of f, column i: vector of v
-                    dst[2 * w] = zr[p][h][k];
-                    dst[2 * w + 1] = zi[p][h][k];
+                    zr[p][h][k] = row_sum(zr[p][h][k]);
+                    zi[p][h][k] = row_sum(zi[p][h][k]);
                 }
-    }
-    __syncthreads();
-    for (int w = threadIdx.x; w < W; w += blockDim.x) {
-        double t = 0;
+        if ((lane & 12) == 0) {
+            float *dst = red + row * wgrad_row(W);
+#pragma unroll
+            for (int p = 0; p < NP; p++)
+#pragma unroll
+                for (int h = 0; h < H; h++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const int w = (p * 4 + i) * CH + 4 * h + k;   // row k: channel of f, column i: vector of v
+                        dst[2 * w] = zr[p][h][k];
+                        dst[2 * w + 1] = zi[p][h][k];
+                    }
+        }
+        __syncthreads();
+        for (int w = lane; w < W; w += blockDim.x) {
+            double t = tot[w];
 #pragma unroll 4
-        for (int q = 0; q < rows; q++) t += (double)wgrad_lds[q * wgrad_row(W) + w];
-        part[(size_t)(P0 * 4 * CH * 2 + w) * gridDim.x + blockIdx.x] = t;
+            for (int q = 0; q < rows; q++) t += (double)red[q * wgrad_row(W) + w];
+            tot[w] = t;
+        }
+        __syncthreads();   // red has been read
     }
+    for (int w = threadIdx.x; w < W; w += blockDim.x) part[(size_t)(P0 * 4 * CH * 2 + w) * gridDim.x + blockIdx.x] = tot[w];
 }
 // paths per group: the sums take 2 CH registers per path, the transports held
 // beside them 24; one more path per group spills (CH = 16: 83 us with three), and

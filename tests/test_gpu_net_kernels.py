@@ -3,7 +3,8 @@ the CPU oracle's layers: the even-odd network with per-thread links (1 and 2
 right-hand sides) and links shared in LDS (3 and more), workgroups of 64, 128
 and 256 threads, last workgroups partly empty and right-hand-side counts that
 do not divide a wavefront; the gradient on lattices that do not fill its last
-workgroup and on one that takes its 256-thread form.
+workgroup, on one that takes its 256-thread form and on one whose workgroups go
+through more rounds of sites than their FP32 sums hold (9).
 
 Tolerances: everything is FP32 arithmetic on FP32 data, so the network agrees
 to a few roundings of its about 100-term sums (2e-6, as for the other FP32
@@ -45,7 +46,8 @@ def test_net_eo_launch_shapes(q, L, nrhs, ch):
             assert rel(got[r], oracle_eo(srcs[r], Ub, L, W1, W2, adjoint)) <= 2e-6, (adjoint, r)
 
 
-@pytest.mark.parametrize("L,ch", [((6, 4, 6, 6), 4), ((6, 4, 6, 6), 16), ((4, 4, 6, 10), 8), ((16, 12, 16, 16), 8)])
+@pytest.mark.parametrize("L,ch", [((6, 4, 6, 6), 4), ((6, 4, 6, 6), 16), ((4, 4, 6, 10), 8), ((16, 12, 16, 16), 8),
+                                  ((24, 22, 24, 18), 16)])
 @pytest.mark.parametrize("prec", ["SINGLE", "DOUBLE"])
 def test_net_gradient_launch_shapes(q, L, ch, prec):
     print(f"gradient L={L} ch={ch} {prec}", flush=True)
