@@ -195,8 +195,14 @@ __global__ __launch_bounds__(kT) QKX_NET_REGS void eo_out_kernel(S in, S out, Ga
     out.store(e, o);
 }
 
-// Links are shared from this many right-hand sides on.
-constexpr int kEoShareMin = 3;
+// Links are shared from this many right-hand sides on.  With 4 hidden channels
+// the kernels are light enough to run five wavefronts per SIMD with a thread's own
+// links, which few right-hand sides' workgroups, each with the links of many sites
+// in LDS, do not reach: 16^3x32 FP16, shared / own: 3 RHS 77 / 53 us, 5 89 / 69,
+// 6 95 / 80 (FP64 129 / 117); 24^4 FP16: 3 RHS 148 / 107, 6 202 / 192 (FP64 336 / 325).
+// With 8 channels: 16^3x32 4 RHS 121 / 105, 24^4 4 RHS 216 / 225, 20^3x44 (FP32)
+// 6 RHS 371 / 394.
+constexpr int eo_share_min(int ch) { return ch == 4 ? 7 : 3; }
 // threads per workgroup: 64 while larger ones would leave SIMDs without a
 // wavefront; 128 for few right-hand sides, whose workgroups hold many sites'
 // links (656 B a site; 42 sites of 3 RHS take 28 KB)
@@ -235,7 +241,7 @@ int launch_eo(qkx_net_s *n, qkx_spinor_s *out, const qkx_spinor_s *in, const qkx
         a.dnc = make_fastdiv(a.nc);
         a.units = a.g.Vh * a.nc;
         const int bs = eo_block(a.units, a.nc);
-        const bool share = a.nc >= kEoShareMin;
+        const bool share = a.nc >= eo_share_min(CH);
         a.upb = share ? bs / a.nc * a.nc : bs;
         const size_t lds = share ? (size_t)(a.upb / a.nc) * kSiteStride * sizeof(float) : 0;
         int nb = (a.units + a.upb - 1) / a.upb;

@@ -1,10 +1,10 @@
 """Learned preconditioner kernels at the edges of their launch shapes, against
-the CPU oracle's layers: the even-odd network with per-thread links (1 and 2
-right-hand sides) and links shared in LDS (3 and more), workgroups of 64, 128
-and 256 threads, last workgroups partly empty and right-hand-side counts that
-do not divide a wavefront; the gradient on lattices that do not fill its last
-workgroup, on one that takes its 256-thread form and on one whose workgroups go
-through more rounds of sites than their FP32 sums hold (9).
+the CPU oracle's layers: the even-odd network with per-thread links (up to 2
+or 6 right-hand sides, by hidden channels) and links shared in LDS, workgroups
+of 64, 128 and 256 threads, last workgroups partly empty and right-hand-side
+counts that do not divide a wavefront; the gradient on lattices that do not fill
+its last workgroup, on one that takes its 256-thread form and on one whose
+workgroups go through more rounds of sites than their FP32 sums hold (9).
 
 Tolerances: everything is FP32 arithmetic on FP32 data, so the network agrees
 to a few roundings of its about 100-term sums (2e-6, as for the other FP32
@@ -27,8 +27,10 @@ def _links(q, L, seed):
 
 
 @pytest.mark.parametrize("L,nrhs,ch", [((4, 6, 4, 6), 1, 4), ((4, 6, 4, 6), 2, 16), ((4, 6, 4, 6), 5, 4),
-                                       ((6, 4, 6, 4), 7, 8), ((6, 4, 6, 4), 16, 4), ((16, 12, 16, 16), 6, 4),
-                                       ((20, 16, 20, 16), 3, 4), ((24, 24, 24, 20), 1, 4)])
+                                       ((6, 4, 6, 4), 7, 8), ((6, 4, 6, 4), 6, 4), ((6, 4, 6, 4), 7, 4),
+                                       ((6, 4, 6, 4), 3, 8), ((6, 4, 6, 4), 16, 4), ((16, 12, 16, 16), 6, 4),
+                                       ((20, 16, 20, 16), 3, 4), ((20, 16, 20, 16), 3, 8),
+                                       ((24, 24, 24, 20), 1, 4)])
 def test_net_eo_launch_shapes(q, L, nrhs, ch):
     print(f"N_e L={L} nrhs={nrhs} ch={ch}", flush=True)
     u32, Ub = _links(q, L, 17)
