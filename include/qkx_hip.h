@@ -122,7 +122,10 @@ int  qkx_prof_reset(void);
 /* Launch shape of the hopping kernel: workgroup size (64/128/256), whether
  * workgroups are remapped so that each XCD walks a contiguous site range, and
  * the software-pipeline depth (1 or 2 hops in flight) of the FP64 and of the
- * FP32/FP16/BF16 kernels. */
+ * FP32/FP16/BF16 kernels.  With the defaults for FP64 (256 threads, depth 2) and
+ * a site order other than 1, hops of one FP64 right-hand side on at most 131,072
+ * output sites take a form with a site's directions on eight wavefronts where
+ * that was measured faster; its results are the same bits. */
 int  qkx_set_tuning(int xcd_remap, int block, int depth64, int depth32);
 /* Order in which the hopping kernels walk the sites of a parity.  1: blocked
  * -- x, then blocks of up to 8 y rows and up to 8 t slices, then z -- so that

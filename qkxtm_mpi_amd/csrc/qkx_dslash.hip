@@ -1624,12 +1624,46 @@ bool share_links_for(int nrhs, long units)
 // 0: checkerboard index order; 1: blocked walk (HopTrav) for every hop;
 // 2: blocked walk where hop_trav's rules say so
 int g_site_order = QKX_SITE_ORDER_DEFAULT;
-// FP64 single-RHS hops of at most this many output sites split each site's
-// directions over eight wavefronts (hop_split_kernel).  tm 13.3 -> 11.6 us at
-// 12^3x32 and 31.4 -> 27.6 us at 16^3x32 (131,072 sites); even-odd normal operator
-// 81.3 -> 74.9 us there (65,536 sites a hop) and equal (57.3 us) at 16^3x24.  Beyond,
-// one thread per site fills the SIMDs and has the half spinors in registers.
-constexpr int kSplitSites = 131072;
+// FP64 single-RHS hops that split each site's directions over eight wavefronts
+// (hop_split_kernel).  hop_kernel needs more than 256 registers in FP64: one
+// wavefront to a SIMD, 65,536 sites to a round of the 1024 SIMDs, and a round
+// takes nearly as long with few sites as with many.  The split form's time grows
+// with the sites, so it wins except where hop_kernel's round is nearly full.
+// us, hop_kernel / split, 18-real links:
+//   half lattice  sites   one hop        even-odd normal operator
+//                 32,768  10.9 /  9.1    47.7 / 38.6
+//                 45,056  12.1 / 12.6    54.3 / 52.8
+//                 53,248  13.5 / 15.2    60.4 / 63.3
+//                 61,440  15.2 / 16.3    67.1 / 68.0
+//                 64,512  17.2 / 17.4    75.0 / 73.4
+//                 81,920  23.8 / 21.3   101   / 84.9
+//   full lattice  sites   tm             iteration of qkx_cg
+//                 40,960  10.2 /  9.5    41.4 / 40.9
+//                 49,152  10.6 / 10.0    43.9 / 45.3
+//                 57,344  11.2 / 11.7    47.5 / 51.6
+//                 64,512  12.1 / 13.3    53.1 / 54.6
+//                 73,728  16.9 / 15.0    71.0 / 63.3
+//                 98,304  18.9 / 18.2    77.2 / 75.6
+//                122,880  23.7 / 22.3    86.6 / 93.8
+// (12-real links at 49,152 sites: one hop 11.1 / 11.2, normal operator 50.5 / 47.8).
+// The full-lattice lines are of lattices whose y extent 8 divides.  With smaller
+// blocks of y rows hop_kernel's walk reuses less, and the split form wins further:
+// tm at 20x20x10x16 13.7 / 12.6, 20^3x14 26.5 / 21.4.  Above 131,072 sites the
+// rounds even out and hop_kernel has the half spinors in registers.
+constexpr int kHopRound = 65536, kSplitSites = 2 * kHopRound;
+// sums: partial sums are asked for, of which the split form leaves four times as
+// many to the kernels that add them
+bool split_hop(const Geom &g, int par_out, bool recon12, bool sums)
+{
+    const int sites = par_out < 0 ? g.V : g.Vh, L1 = g.L[1];
+    if (sites > kSplitSites) return false;
+    if (par_out >= 0) return sites <= kHopRound / 16 * (recon12 ? 12 : 11) || sites > kHopRound / 16 * 15;
+    if (sites <= kHopRound) return (L1 % 8 && L1 % 7) || sites <= kHopRound / 16 * (sums ? 11 : 12);
+    return !(sums && L1 % 8 == 0 && sites > kHopRound / 2 * 3);
+}
+// The split form has one launch shape and walks in checkerboard order: a caller
+// who sets another shape (qkx_set_tuning) or asks for the blocked walk gets hop_kernel.
+bool split_allowed() { return g_block == 256 && g_depth64 == 2 && g_site_order != 1; }
 #ifndef QKX_STAGE_DEFAULT
 #define QKX_STAGE_DEFAULT 0
 #endif
@@ -1827,11 +1861,12 @@ int launch_hop_t(qkx_spinor_s *out, const qkx_spinor_s *in, const qkx_spinor_s *
             }
         }
     }
-    // small FP64 lattices, unless the autotuner timed this kind or a candidate is being timed
+    // small FP64 lattices, unless the autotuner (mode 2) times this kind
     constexpr bool split64 = std::is_same_v<S, SpinorD> &&
                              (store || std::is_same_v<Fin, CgFin<SpinorD, SpinorD, SpinorD, true>>);
     if constexpr (split64) {
-        if (a.nrhs == 1 && sites_out <= kSplitSites && !g_force && g_autotune != 2) {
+        if (a.nrhs == 1 && !g_force && g_autotune != 2 && split_allowed() &&
+            split_hop(a.g, par_out, U->recon == QKX_RECON_12, !store || norm_partial)) {
             int nbh = (a.g.Vh + 63) / 64;   // blocks per parity
             a.nblk8 = 0;
             if (g_xcd_remap && nbh >= 64) {

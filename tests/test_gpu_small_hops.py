@@ -1,19 +1,17 @@
 """FP64 hops of small lattices, whose directions run on eight wavefronts,
-against the one-thread-per-site kernel (which the autotuner, asked to tune
-every launch, selects): every operator form, both bases and link storages, on
-lattices whose parity does not fill its last 64 sites and on one that takes
-the XCD-remapped grid.  Both kernels form and add the same FP64 products in
-the same order; the compiler may contract one product and sum differently, so
-the results may differ in the last bits of a hop's 144-term sums (1e-15)."""
+against the one-thread-per-site kernel, which a caller gets by asking for the
+blocked walk or for a launch shape: every operator form, both bases and link
+storages, on lattices whose parity does not fill its last 64 sites and on some
+that take the XCD-remapped grid, with and without padding workgroups.  Both
+kernels form and add the same FP64 products in the same order: the same bits,
+and the bits of a batch's members."""
 import numpy as np
 import pytest
-
-from refops import rel
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("L", [(4, 4, 4, 4), (6, 4, 6, 4), (4, 6, 10, 6), (8, 8, 8, 16)])
+@pytest.mark.parametrize("L", [(4, 4, 4, 4), (6, 4, 6, 4), (4, 6, 10, 6), (8, 8, 8, 16), (10, 8, 8, 14)])
 @pytest.mark.parametrize("recon", ["RECON_18", "RECON_12"])
 def test_split_hop_matches_one_thread_per_site(q, L, recon):
     print(f"split hops L={L} {recon}", flush=True)
@@ -33,12 +31,17 @@ def test_split_hop_matches_one_thread_per_site(q, L, recon):
     }
     got = {}
     try:
-        for mode in (2, 0):
-            q.set_autotune(mode)
-            for name, run in ops.items():
+        for name in ("split", "walk", "shape"):
+            q.set_site_order(1 if name == "walk" else 2)
+            q.set_tuning(block=128 if name == "shape" else 256)
+            for op, run in ops.items():
                 run()
-                got[name, mode] = (f if name == "normal_odd" else y).download()
+                got[name, op] = (f if op == "normal_odd" else y).download()
     finally:
-        q.set_autotune(1)
-    for name in ops:
-        assert rel(got[name, 0], got[name, 2]) <= 1e-15, name
+        q.set_site_order(2)
+        q.set_tuning()
+    for op in ops:
+        assert np.array_equal(got["split", op], got["walk", op]) and np.array_equal(got["split", op], got["shape", op]), op
+    b, c = q.Spinor(L, host=np.stack([psi, 2 * psi]), nrhs=2), q.Spinor(L, nrhs=2)
+    c.tm(b, u, p)
+    assert np.array_equal(c.download_rhs(0), got["split", "tm"])
