@@ -153,7 +153,8 @@ int  qkx_set_batch_link_sharing(int on);
  * storage, right-hand sides, lattice sites, full or half lattice, dagger,
  * xpay input, basis) it times the candidate launch shapes -- workgroup size
  * (256 or 128 threads), links shared through LDS (batches of 3-16 RHS),
- * pipeline depth -- on scratch fields of that kind and keeps the fastest for
+ * pipeline depth, and the form of small FP64 lattices (reported as block=512)
+ * -- on scratch fields of that kind and keeps the fastest for
  * every later launch of the kind.  Each shape computes every output site
  * with the same arithmetic: the same bits for FP16 and FP64 fields; FP32 and
  * BF16 batches with shared links may round a contracted product-sum
