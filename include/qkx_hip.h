@@ -150,8 +150,8 @@ int  qkx_set_neighbour_staging(int mode);
  * The hop results are identical. */
 int  qkx_set_batch_link_sharing(int on);
 /* The hop autotuner: on the first launch of a kind (spinor and link
- * storage, right-hand sides, lattice sites, full or half lattice, dagger,
- * xpay input, basis) it times the candidate launch shapes -- workgroup size
+ * storage, right-hand sides, lattice, full or half lattice, dagger, xpay
+ * input, basis, site order) it times the candidate launch shapes -- workgroup size
  * (256 or 128 threads), links shared through LDS (batches of 3-16 RHS),
  * pipeline depth, and the form of small FP64 lattices (reported as block=512)
  * -- on scratch fields of that kind and keeps the fastest for

@@ -16,6 +16,7 @@
 // reference's conventions and are necessarily identical to it.
 #include "qkx_internal.h"
 #include <algorithm>
+#include <array>
 #include <map>
 #include <string>
 #include <type_traits>
@@ -1684,19 +1685,14 @@ struct HopShape {
     int depth;
 };
 // The autotuner: on the first launch of a kind (spinor and link storage,
-// right-hand sides, output sites, full or half lattice, dagger, xpay input,
-// basis) it times the candidate shapes on scratch fields of that kind and
-// caches the fastest for every later launch of the kind.
+// right-hand sides, lattice, full or half lattice, dagger, xpay input, basis,
+// and the site order, which with the lattice sets the walk) it times the
+// candidate shapes on scratch fields of that kind and caches the fastest for
+// every later launch of the kind.
 struct TuneKey {
-    int sp, gp, gr, nrhs, sites, full, dag, aux, basis;
-    bool operator<(const TuneKey &o) const
-    {
-        const int x[9] = {sp, gp, gr, nrhs, sites, full, dag, aux, basis};
-        const int y[9] = {o.sp, o.gp, o.gr, o.nrhs, o.sites, o.full, o.dag, o.aux, o.basis};
-        for (int i = 0; i < 9; i++)
-            if (x[i] != y[i]) return x[i] < y[i];
-        return false;
-    }
+    int sp, gp, gr, nrhs, L[4], full, dag, aux, basis, order;
+    std::array<int, 13> all() const { return {sp, gp, gr, nrhs, L[0], L[1], L[2], L[3], full, dag, aux, basis, order}; }
+    bool operator<(const TuneKey &o) const { return all() < o.all(); }
 };
 struct TuneEntry {
     HopShape shape;
@@ -1859,8 +1855,8 @@ int launch_hop_t(qkx_spinor_s *out, const qkx_spinor_s *in, const qkx_spinor_s *
         if (g_force) {
             sh = *g_force;
         } else if (rt == 1 && !g_tuning && !g_no_tune && (g_autotune == 2 || (g_autotune == 1 && a.nrhs > 1))) {
-            const TuneKey key{in->prec, U->prec, U->recon, a.nrhs, sites_out, par_out < 0 ? 1 : 0, dagger,
-                              aux ? 1 : 0, B};
+            const TuneKey key{in->prec, U->prec, U->recon, a.nrhs, {U->L[0], U->L[1], U->L[2], U->L[3]},
+                              par_out < 0 ? 1 : 0, dagger, aux ? 1 : 0, B, g_site_order};
             auto it = g_tuned.find(key);
             if (it == g_tuned.end()) {
                 tune_hop<S, G, B>(key, out, in, aux, U, dagger, par_out, e, sh, share_ok && a.nrhs >= kShareMinRhs,
@@ -2157,10 +2153,11 @@ std::string tune_report()
         const TuneEntry &t = kv.second;
         char line[256];
         snprintf(line, sizeof line,
-                 "spinor_prec=%d gauge_prec=%d recon=%d nrhs=%d sites=%d full=%d dagger=%d xpay=%d basis=%d : "
-                 "block=%d share=%d depth=%d %.2f us (default %.2f us)\n",
-                 k.sp, k.gp, k.gr, k.nrhs, k.sites, k.full, k.dag, k.aux, k.basis, t.shape.block, t.shape.share,
-                 t.shape.depth, t.us, t.default_us);
+                 "spinor_prec=%d gauge_prec=%d recon=%d nrhs=%d sites=%d lattice=%dx%dx%dx%d full=%d dagger=%d xpay=%d "
+                 "basis=%d order=%d : block=%d share=%d depth=%d %.2f us (default %.2f us)\n",
+                 k.sp, k.gp, k.gr, k.nrhs, k.L[0] * k.L[1] * k.L[2] * k.L[3] / (k.full ? 1 : 2), k.L[0], k.L[1],
+                 k.L[2], k.L[3], k.full, k.dag, k.aux, k.basis, k.order, t.shape.block, t.shape.share, t.shape.depth,
+                 t.us, t.default_us);
         r += line;
     }
     return r;

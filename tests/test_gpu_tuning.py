@@ -118,3 +118,24 @@ def test_tuner_knows_the_small_lattice_form(q):
     print(report, flush=True)
     assert report.count("\n") == 1 and "block=512" in report
     assert np.array_equal(out[0], out[2])
+
+
+def test_tuned_kinds_keep_lattices_and_site_orders_apart(q):
+    """Lattices of one volume walk their sites in different blocks, and so do site
+    orders: each is a kind of its own to the tuner."""
+    P, nrhs = q.HALF, 8
+    try:
+        q.set_autotune(1)
+        for n, (L, order) in enumerate([((8, 8, 8, 16), 2), ((16, 8, 8, 8), 2), ((16, 8, 8, 8), 1)], 1):
+            q.set_site_order(order)
+            u = q.Gauge(L, P, q.RECON_12, -1)
+            u.convert_from(q.Gauge(L, boundaryT=-1, host=q.gen_gauge(L, 0.3, 5)))
+            x, y = q.Spinor(L, P, nrhs=nrhs), q.Spinor(L, P, nrhs=nrhs)
+            x.gaussian(7)
+            y.tm(x, u, q.params(L, 0.1632, 0.004, 1, -1))
+            report = q.autotune_report()
+            print(report, flush=True)
+            assert report.count("\n") == n and f"lattice={'x'.join(map(str, L))} " in report
+    finally:
+        q.set_site_order(2)
+        q.set_autotune(1)
