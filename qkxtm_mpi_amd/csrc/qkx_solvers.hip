@@ -306,9 +306,12 @@ __global__ __launch_bounds__(kThreads) void cg_dir_small_kernel(double2 *p, cons
     if (flag || i >= n12) return;
     p[i] = make_double2(rv.x + beta * pv.x, rv.y + beta * pv.y);
 }
-// At most this many sites: 768 workgroups, each summing 2 x 256 partials; with
-// more, one thread per site fills the CUs and repeats the sums less often.
-constexpr int kDirSmallSites = 16384;
+// At most this many sites: 480 workgroups, each summing the partials; with more,
+// one thread per site repeats the sums twelve times less often.  us an iteration,
+// per site / per complex number: full lattice 4,096 sites 20.7 / 19.1, 8,192 20.6 /
+// 20.2, 13,824 23.2 / 23.9, 20,736 28.2 / 29.7; even-odd FP64 4,096 30.6 / 29.7,
+// 8,192 33.5 / 31.0, 10,368 35.7 / 35.6, 20,736 42.1 / 44.3.
+constexpr int kDirSmallSites = 10240;
 
 // every workgroup sums v[0..n) with block_sum_array and writes its result
 __global__ __launch_bounds__(kThreads) void block_sum_probe_kernel(const double *v, int n, double *out)
