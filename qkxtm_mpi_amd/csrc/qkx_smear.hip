@@ -759,11 +759,15 @@ void launch_march(const GaussMarch &m, const MarchGrid &r)
     else if (r.loads <= 6) hipLaunchKernelGGL(gauss_march_kernel<6>, r.grid, dim3(256), r.lds, qkx::g_stream, m);
     else hipLaunchKernelGGL(gauss_march_kernel<12>, r.grid, dim3(256), r.lds, qkx::g_stream, m);
 }
-// A step of at least this many (site, right-hand side) units marches.  24 planes
-// in a row are a chain that needs enough workgroups beside it: 10 steps at
-// 16^3x32 (131,072 units) 318 -> 260 us, 30 steps of a 24^3 slice with 12
-// right-hand sides (165,888) 781 -> 760 us; a 48^3 slice with one (110,592) 709
-// -> 753 us, 8^3x16 with 12 (98,304) 269 -> 294 us.
+// A step of at least this many (site, right-hand side) units marches: 24 planes in
+// a row are a chain that needs enough workgroups beside it.  The line is where the
+// two forms cross on average; a shape near it may be either way by a few percent.
+// us a step, per unit / marching:
+//   16^3x32, 1 RHS (131,072)  29.6 / 24.8    slice  48^3, 1 RHS (110,592)  23.6 / 25.1
+//   14^3x24, 2     (131,712)  29.7 / 23.6           32^3, 4     (131,072)  22.8 / 19.4
+//   12^3x20, 4     (138,240)  23.4 / 24.0           28^3, 6     (131,712)  22.4 / 23.3
+//   12^3x24, 4     (165,888)  25.0 / 23.9           24^3, 10    (138,240)  22.4 / 23.2
+//   8^3x16, 12      (98,304)  26.9 / 29.4           24^3, 13    (179,712)  27.2 / 25.9
 constexpr long kMarchUnits = 131072;
 // its link elements are indexed with 32 bits
 constexpr long kMarchSites = ((1L << 31) - 1) / 27;

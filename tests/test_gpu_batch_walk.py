@@ -1,13 +1,15 @@
 """Batched hops on a lattice whose t slice exceeds an XCD's L2 walk the sites
 in blocks by default: the same bits as in checkerboard order, for 8 (the
-fewest) and 12 right-hand sides, with extents that 8 does not divide."""
+fewest) and 12 right-hand sides in every storage, with extents that 8 does not
+divide."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("prec,nrhs", [("HALF", 12), ("HALF", 8), ("BF16", 12)])
+@pytest.mark.parametrize("prec,nrhs", [("HALF", 12), ("HALF", 8), ("BF16", 12), ("SINGLE", 8), ("SINGLE", 12),
+                                       ("DOUBLE", 8)])
 def test_batch_walk_identical(q, prec, nrhs):
     L = (20, 20, 22, 6)
     print(f"batch walk L={L} {prec} nrhs={nrhs}", flush=True)
