@@ -1647,10 +1647,12 @@ int g_site_order = QKX_SITE_ORDER_DEFAULT;
 //                 98,304  18.9 / 18.2    77.2 / 75.6
 //                122,880  23.7 / 22.3    86.6 / 93.8
 // (12-real links at 49,152 sites: one hop 11.1 / 11.2, normal operator 50.5 / 47.8).
-// The full-lattice lines are of lattices whose y extent 8 divides.  With smaller
-// blocks of y rows hop_kernel's walk reuses less, and the split form wins further:
-// tm at 20x20x10x16 13.7 / 12.6, 20^3x14 26.5 / 21.4.  Above 131,072 sites the
-// rounds even out and hop_kernel has the half spinors in registers.
+// The full-lattice lines are of lattices whose y extent 8 divides and whose rows
+// have 12 sites or more.  With smaller blocks hop_kernel's walk reuses less, and the
+// split form wins further: tm at 20x20x10x16 13.7 / 12.6, 20^3x14 26.5 / 21.4, hop
+// at 8x16x16x32 14.3 / 13.5.  At exactly one or two rounds hop_kernel takes 12.4 or
+// 17.5 us, 94 or 108 an iteration, by where its workgroups land.  Above 131,072
+// sites the rounds even out and hop_kernel has the half spinors in registers.
 constexpr int kHopRound = 65536, kSplitSites = 2 * kHopRound;
 // sums: partial sums are asked for, of which the split form leaves four times as
 // many to the kernels that add them
@@ -1659,8 +1661,9 @@ bool split_hop(const Geom &g, int par_out, bool recon12, bool sums)
     const int sites = par_out < 0 ? g.V : g.Vh, L1 = g.L[1];
     if (sites > kSplitSites) return false;
     if (par_out >= 0) return sites <= kHopRound / 16 * (recon12 ? 12 : 11) || sites > kHopRound / 16 * 15;
-    if (sites <= kHopRound) return (L1 % 8 && L1 % 7) || sites <= kHopRound / 16 * (sums ? 11 : 12);
-    return !(sums && L1 % 8 == 0 && sites > kHopRound / 2 * 3);
+    if (g.L[0] < 12 || (L1 % 8 && L1 % 7)) return true;
+    if (sites < kHopRound) return sites <= kHopRound / 16 * (sums ? 11 : 12);
+    return !(sums && L1 % 8 == 0 && sites > kHopRound / 16 * 24 && sites <= kHopRound / 16 * 30);
 }
 // The split form has one launch shape and walks in checkerboard order: a caller
 // who sets another shape (qkx_set_tuning) or asks for the blocked walk gets hop_kernel.
@@ -1711,8 +1714,10 @@ thread_local int g_no_tune = 0;     // callers that must not allocate (scratch f
 //    parity) moves more than an XCD's 4 MB L2 holds, so that in plain order the
 //    t neighbours are fetched again for every slice: 12-RHS even-odd normal
 //    operator 2372 -> 2275 us in FP16 and 4140 -> 3974 us in FP32 at 32^3x64,
-//    729 -> 718 us in FP16 at 24^3x48; at 16^3x32 (2.9 MB a slice) it changes
-//    nothing, and with 3 right-hand sides it costs 2-3%.
+//    729 -> 718 us in FP16 at 24^3x48, 1112 -> 1061 in BF16 at 32^4, 8 right-hand
+//    sides in FP64 at 32^3x16 1483 -> 1343.  Just above 4 MB a slice it gives
+//    nothing (FP64 and FP32 at 12x24^3 and 20^3x32: -2 to +4%, FP16 and BF16 -3 to
+//    +2%), and with 3 right-hand sides it costs 2-3%.
 constexpr double kTravAutoBytes = 700.0;
 constexpr int kTravAutoRhs = 8;
 constexpr double kTravL2 = 4.0e6;
